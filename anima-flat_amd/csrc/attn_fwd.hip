@@ -77,6 +77,8 @@
 
 #include "attn_fwd.h"
 #include "attn_fwd_d384.h"
+#include "attn_fwd_ks.h"
+#include "attn_fwd_wave.h"
 #include "tile_io.h"
 
 namespace aa {
@@ -87,7 +89,6 @@ static_assert(kWaves * kQPerWave == kQPerWg, "work item size");
 constexpr int kStages = 4;                   // K/V ring depth (4 x 32 KB)
 constexpr int kLead = kStages - 1;           // tile t + kLead is fetched during tile t
 constexpr uint32_t kStageBytes = 2u * kTileElems * sizeof(bf16);  // K tile, then V tile
-constexpr uint32_t kVOff = kTileElems * sizeof(bf16);             // V tile in a stage
 
 // K/V tile DMA of one wave into the K and V line tiles of a ring stage
 // (tile_io.h). A DMA instruction fills one 1 KB block = 8 rows x 64 d from 8
@@ -157,384 +158,25 @@ struct KVDma {
     }
   }
 
+  // FwdWave::tile's hooks: instruction i goes out in slot 4 i + 3 (and the
+  // workgroup waits for the job at the tile's top, not in its slots).
+  template <int B, class W>
+  __device__ __forceinline__ void mask(W& w, int kb, int klen) const { w.template mask<B>(kb, klen); }
+  template <int g>
+  __device__ __forceinline__ void first_slot() const {}
+  template <int g, bool NEXT>
+  __device__ __forceinline__ void before_slot() const {}
+  template <int g, bool NEXT>
+  __device__ __forceinline__ void after_slot() const {
+    if constexpr ((g & 3) == 3 && g < 32) issue<(g >> 2)>();
+  }
+
   // DMA instruction i of the job: 0-3 the K blocks, 4-7 the V blocks.
   template <int i>
   __device__ __forceinline__ void issue() const {
     constexpr uint32_t off = (i < 4 ? 0u : kVOff) + (uint32_t)(i & 3) * 1024u;
     if constexpr (i < 4) dma16_sva(kbase, ko[i & 3], dst + off);
     else dma16_sva(vbase, vo[i & 3], dst + off);
-  }
-};
-
-// Operand reads ahead of their MFMA: K operands (each feeds the two MFMAs of
-// a pair of slots) are read kKPf pairs ahead, V^T operands kVPf pairs ahead
-// into a queue one entry longer than that needs (a V^T operand stays
-// allocated for one slot after its last MFMA).
-constexpr int kKPf = 2, kKQ = kKPf + 1;
-constexpr int kVPf = 2, kVQ = kVPf + 2;
-constexpr int kread_slot(int j) { return j < kKPf ? 0 : 2 * (j - kKPf); }
-constexpr int vread_slot(int pp) { return 32 + 2 * (pp - kVPf); }
-// P unit u (2 scores of query block (u >> 2) & 1, key chunk u >> 3) starts in
-// slot 3u / 2 and ends two slots later (slots 0-48); the P operand of chunk c4
-// is first used in slot 32 + 8 c4, after its last unit. Max steps of the next
-// tile: slots 48-63.
-constexpr int exp_slot(int u) { return (3 * u) / 2; }
-constexpr int kMaxSlot0 = 48;
-// DMA instruction i of the tile's job: slot 4 i + 3.
-constexpr int dma_slot(int i) { return 4 * i + 3; }
-
-// O^T += V^T P^T with O in AGPRs, as inline asm: the builtin would follow the
-// function-wide choice of one register file for every MFMA accumulator, and S
-// must stay in VGPRs for the softmax. O is only read or written by VALU code
-// behind fence_o(), and the A/B operands are read when the MFMA issues.
-__device__ __forceinline__ void mfma_pv(f32x16& acc, bf16x8 a, bf16x8 b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
-__device__ __forceinline__ void keep_alive(bf16x8 v) { asm volatile("" ::"v"(v)); }
-// Row sums (the accumulator and the 0/1 selector in AGPRs, as for O).
-__device__ __forceinline__ void mfma_rowsum(f32x4& acc, bf16x8 sel, bf16x8 p) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "a"(sel), "v"(p));
-}
-
-// Per-wave state and work: 64 queries (blocks qb = 0, 1 of 32), their Q^T
-// operands, O^T accumulators and running softmax statistics.
-struct FwdWave {
-  bf16x8 qreg[2][8];  // Q^T (qb, kk): lane holds Q[32 qb + li][16 kk + 8 hh + 0..7]; AGPRs
-  f32x16 o[4][2];     // O^T (dt, qb): d = 32 dt + rows, query 32 qb + li; AGPRs
-  f32x16 s[2][2][2];  // S^T (buffer, kb, qb): keys 32 kb + rows of the tile, query 32 qb + li
-  bf16x8 pb[4][2];    // P^T (c4, qb): keys 16 c4 + .. of the tile, in accumulator order
-  float m_raw[2];     // running max of query 32 qb + li, raw score units
-  float mt[2];        // row max of the next tile (raw)
-  f32x4 lsum[2];      // row sum of query 32 qb + li (all four elements), by MFMA
-  bf16x8 sel;         // 0/1 selector: the A operand of the row-sum MFMA
-  float c, thr_raw;
-  int li, hh;
-  uint32_t kb4[4];  // LDS byte address of this lane's K operand reads in the next tile's K
-                    // (line_k_rd(lane, j)); advanced one stage per tile
-  uint32_t vb2[2];  // ... of its V^T operand reads in this tile's V (line_v_tr(lane, p))
-
-  // LDS read bases start at ring stage 0 (tile 0).
-  __device__ __forceinline__ void setup(int lane, float c_, uint32_t ring) {
-    li = lane & 31;
-    hh = lane >> 5;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) kb4[j] = ring + 2u * (uint32_t)line_k_rd(lane, j);
-    vb2[0] = ring + kVOff + 2u * (uint32_t)line_v_tr(lane, 0);
-    vb2[1] = ring + kVOff + 2u * (uint32_t)line_v_tr(lane, 1);
-    c = c_;
-    thr_raw = kRescaleThreshold / c;
-    // Zeros pinned into AGPRs, the file every later MFMA keeps O in.
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
-        o[dt][qb] = f32x16{};
-        asm volatile("" : "+a"(o[dt][qb]));
-      }
-    m_raw[0] = m_raw[1] = -INFINITY;
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
-      lsum[qb] = f32x4{};
-      asm volatile("" : "+a"(lsum[qb]));
-    }
-    // Row sums by v_mfma_f32_16x16x32_bf16 with the P^T operand as B: in that
-    // shape lane l's 8 values are B[k = 8 (l / 16) + i][n = l % 16], i.e.
-    // query n (+16 for odd l / 16) over one half of the chunk's keys. With
-    // A[m][k] = 1 where bit 2 of m equals bit 3 of k, D[m][n] sums query n
-    // for m % 8 < 4 and query n + 16 otherwise, which puts the row sum of
-    // query li = lane % 32 in all four D values of lane `lane`.
-    {
-      const bf16 one = (bf16)(((lane & 15) >> 2 & 1) == ((lane >> 4) & 1) ? 1.0f : 0.0f);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) sel[i] = one;
-      asm volatile("" : "+a"(sel));
-    }
-  }
-
-  // Q^T operands from this wave's 64 staged rows (two 32-row staging areas),
-  // kept in AGPRs (the MFMA reads its B operand from either file).
-  __device__ __forceinline__ void read_q(const bf16* stage, int lane) {
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-        qreg[qb][kk] = staged_operand(stage + qb * 4096, lane, kk);
-        asm volatile("" : "+a"(qreg[qb][kk]));
-      }
-  }
-
-  // K operand pair j = 8 kb + kk (keys 32 kb .., head-dim 16 kk ..) of the K
-  // tile at kb4.
-  template <int j>
-  __device__ __forceinline__ bf16x8 k_op() const {
-    constexpr int kb = j >> 3, kk = j & 7;
-    return lds_ld16(kb4[kk & 3] + 8192u * (kk >> 2) + 4096u * kb);
-  }
-  // V^T operand pair pp = 4 c4 + dt (d 32 dt .., keys of chunk c4).
-  template <int pp>
-  __device__ __forceinline__ bf16x8 v_op() const {
-    constexpr int c4 = pp >> 2, dt = pp & 3;
-    constexpr uint32_t off = 8192u * (dt >> 1) + 2048u * c4;
-    const s16x4 lo = lds_ld8_tr(vb2[dt & 1] + off);
-    const s16x4 hi = lds_ld8_tr(vb2[dt & 1] + off + 1024u);
-    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-  }
-  // Moves the K / V^T read bases on by `delta` bytes (the next ring stage).
-  __device__ __forceinline__ void advance_k(uint32_t delta) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      kb4[j] += delta;
-      asm volatile("" : "+v"(kb4[j]));
-    }
-  }
-  __device__ __forceinline__ void advance_v(uint32_t delta) {
-    vb2[0] += delta;
-    vb2[1] += delta;
-    asm volatile("" : "+v"(vb2[0]), "+v"(vb2[1]));
-  }
-
-  // Scores of keys at or past klen (tile at key offset kb) to -inf.
-  template <int B>
-  __device__ __forceinline__ void mask(int kb, int klen) {
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kb + 32 * kt + 8 * (r >> 2) + 4 * hh + (r & 3);
-          if (key >= klen) s[B][kt][qb][r] = -INFINITY;
-        }
-  }
-
-  // Max step k (0..15) of S^T buffer B: block kb = k >> 3, query block
-  // qb = k & 1, registers 4 ((k >> 1) & 3) .. + 3, into mx[qb].
-  template <int B, int k>
-  __device__ __forceinline__ void max_step(float (&mx)[2]) const {
-    constexpr int kb = k >> 3, qb = k & 1, r0 = 4 * ((k >> 1) & 3);
-    const f32x16& a = s[B][kb][qb];
-    if constexpr (k < 2) {
-      mx[qb] = max2f(max3f(a[r0], a[r0 + 1], a[r0 + 2]), a[r0 + 3]);
-    } else {
-      mx[qb] = max3f(mx[qb], a[r0], a[r0 + 1]);
-      mx[qb] = max3f(mx[qb], a[r0 + 2], a[r0 + 3]);
-    }
-  }
-
-  // P unit u of S^T buffer B: scores 2 jp, 2 jp + 1 of the P operand (c4, qb),
-  // c4 = u >> 3, qb = (u >> 2) & 1, jp = u & 3, and their sum, in three
-  // stages one slot apart (fma, exp, pack + sum): the stages of consecutive
-  // units share a slot, so no VALU instruction waits on the one before it.
-  // fa / fe carry two units' values between the stages.
-  template <int B, int u>
-  __device__ __forceinline__ void p_fma(const float (&mc)[2], float (&fa)[2][2]) const {
-    constexpr int c4 = u >> 3, qb = (u >> 2) & 1, jp = u & 3;
-    constexpr int kb = c4 >> 1, r = 8 * (c4 & 1) + 2 * jp;
-    fa[u & 1][0] = fmaf(s[B][kb][qb][r], c, -mc[qb]);
-    fa[u & 1][1] = fmaf(s[B][kb][qb][r + 1], c, -mc[qb]);
-    asm volatile("" : "+v"(fa[u & 1][0]), "+v"(fa[u & 1][1]));
-  }
-  template <int u>
-  __device__ __forceinline__ void p_exp(const float (&fa)[2][2], float (&fe)[2][2]) const {
-    fe[u & 1][0] = fast_exp2(fa[u & 1][0]);
-    fe[u & 1][1] = fast_exp2(fa[u & 1][1]);
-    asm volatile("" : "+v"(fe[u & 1][0]), "+v"(fe[u & 1][1]));
-  }
-  template <int u>
-  __device__ __forceinline__ void p_pack(const float (&fe)[2][2]) {
-    constexpr int c4 = u >> 3, qb = (u >> 2) & 1, jp = u & 3;
-    pb[c4][qb][2 * jp] = (bf16)fe[u & 1][0];
-    pb[c4][qb][2 * jp + 1] = (bf16)fe[u & 1][1];
-    // Anchored in its slot: left alone, the compiler sinks the P work next to
-    // its MFMA users.
-    asm volatile("" : "+v"(pb[c4][qb]));
-  }
-  // Row sums of the P operand (c4, qb) on the matrix pipe (see setup): the
-  // VALU alternatives cost the SIMD's vector issue (fp32 adds) or stall the
-  // matrix pipe for half an MFMA each (v_dot2c_f32_bf16).
-  template <int c4, int qb>
-  __device__ __forceinline__ void p_sum() {
-    mfma_rowsum(lsum[qb], sel, pb[c4][qb]);
-  }
-
-  // S^T of the first tile of the range (no other work to interleave).
-  template <int B>
-  __device__ __forceinline__ void qk_first() {
-    bf16x8 kq[kKQ];
-    static_for<0, 32 + 2 * kKPf>([&](auto G) {
-      constexpr int g = decltype(G)::value;
-      static_for<0, 16>([&](auto J) {
-        constexpr int j = decltype(J)::value;
-        if constexpr (kread_slot(j) == g) kq[j % kKQ] = this->template k_op<j>();
-      });
-      if constexpr (g < 32) {
-        constexpr int j = g >> 1, kb = j >> 3, kk = j & 7, qb = g & 1;
-        s[B][kb][qb] = mfma32(kq[j % kKQ], qreg[qb][kk], kk == 0 ? f32x16{} : s[B][kb][qb]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  }
-
-  // Row max of S^T buffer B into mt (no other work).
-  template <int B>
-  __device__ __forceinline__ void max_plain() {
-    float mx[2];
-    static_for<0, 16>([&](auto K) { this->template max_step<B, decltype(K)::value>(mx); });
-    mt[0] = pair_max(mx[0]);
-    mt[1] = pair_max(mx[1]);
-  }
-
-  // One tile t of the slot schedule. S^T of tile t is in buffer SB; with
-  // NEXT, S^T of tile t+1 (its K one ring stage, dstage bytes, past tile t's)
-  // goes to buffer 1 - SB (masked first when its keys end inside it:
-  // mask_next) and, with TRACK, its row max to mt. The DMA job is issued in
-  // its slots.
-  template <int SB, bool NEXT, bool TRACK>
-  __device__ __forceinline__ void tile(uint32_t dstage, bool mask_next, int kb_next, int klen,
-                                       const KVDma& dma) {
-    constexpr int NB = 1 - SB;
-    const float mc[2] = {m_raw[0] * c, m_raw[1] * c};
-    if constexpr (NEXT) advance_k(dstage);
-    bf16x8 kq[kKQ], vq[kVQ];
-    float mx[2];
-    float fa[2][2], fe[2][2];
-    static_for<0, 64>([&](auto G) {
-      constexpr int g = decltype(G)::value;
-      if constexpr (NEXT && g == kMaxSlot0) {
-        if (mask_next) mask<NB>(kb_next, klen);
-      }
-      // Operand reads.
-      if constexpr (NEXT) {
-        static_for<0, 16>([&](auto J) {
-          constexpr int j = decltype(J)::value;
-          if constexpr (kread_slot(j) == g) kq[j % kKQ] = this->template k_op<j>();
-        });
-      }
-      static_for<0, 16>([&](auto P) {
-        constexpr int pp = decltype(P)::value;
-        if constexpr (vread_slot(pp) == g) vq[pp % kVQ] = this->template v_op<pp>();
-      });
-      // The slot's MFMA.
-      if constexpr (g < 32) {
-        if constexpr (NEXT) {
-          constexpr int j = g >> 1, kb = j >> 3, kk = j & 7, qb = g & 1;
-          s[NB][kb][qb] = mfma32(kq[j % kKQ], qreg[qb][kk], kk == 0 ? f32x16{} : s[NB][kb][qb]);
-        }
-      } else {
-        constexpr int op = g - 32, pp = op >> 1, c4 = pp >> 2, dt = pp & 3, qb = op & 1;
-        mfma_pv(o[dt][qb], vq[pp % kVQ], pb[c4][qb]);
-        if constexpr (dt == 2) this->template p_sum<c4, qb>();
-      }
-
-      // P units of tile t, three stages per unit.
-      static_for<0, 32>([&](auto U) {
-        constexpr int u = decltype(U)::value;
-        if constexpr (exp_slot(u) == g) this->template p_fma<SB, u>(mc, fa);
-        if constexpr (exp_slot(u) + 1 == g) this->template p_exp<u>(fa, fe);
-        if constexpr (exp_slot(u) + 2 == g) this->template p_pack<u>(fe);
-      });
-      // Row max of tile t+1.
-      if constexpr (NEXT && TRACK && g >= kMaxSlot0) {
-        this->template max_step<NB, g - kMaxSlot0>(mx);
-        asm volatile("" : "+v"(mx[0]), "+v"(mx[1]));
-      }
-      // DMA.
-      static_for<0, 8>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-        if constexpr (dma_slot(i) == g) dma.template issue<i>();
-      });
-      // The operands of the previous slot's inline-asm MFMA stay allocated to
-      // the end of this slot: the compiler does not see that MFMA still
-      // reading them and would hand their registers to this slot's VALU
-      // results, whose writes would then wait for it.
-      if constexpr (g > 32) {
-        constexpr int op = g - 33, pp = op >> 1, c4 = pp >> 2, dt = pp & 3, qb = op & 1;
-        keep_alive(vq[pp % kVQ]);
-        if constexpr (dt == 3) keep_alive(pb[c4][qb]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    keep_alive(vq[15 % kVQ]);
-    keep_alive(pb[3][1]);
-    advance_v(dstage);
-    if constexpr (NEXT && TRACK) {
-      mt[0] = pair_max(mx[0]);
-      mt[1] = pair_max(mx[1]);
-    }
-  }
-
-  // Keeps O in AGPRs up to this point and orders the VALU code that follows
-  // after every MFMA that wrote it.
-  __device__ __forceinline__ void fence_o() {
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3"
-                 : "+a"(o[0][0]), "+a"(o[1][0]), "+a"(o[2][0]), "+a"(o[3][0]), "+a"(o[0][1]),
-                   "+a"(o[1][1]), "+a"(o[2][1]), "+a"(o[3][1]), "+a"(lsum[0]), "+a"(lsum[1]));
-  }
-
-  // Lazy rescale for the next tile's max mt: m is raised (and O and l scaled
-  // down) only where mt exceeds it by more than thr_raw.
-  __device__ __forceinline__ void update_max() {
-    const bool n0 = mt[0] > m_raw[0] + thr_raw;
-    const bool n1 = mt[1] > m_raw[1] + thr_raw;
-    if (__builtin_amdgcn_ballot_w64(n0 || n1)) {
-      const float mn0 = n0 ? mt[0] : m_raw[0];
-      const float mn1 = n1 ? mt[1] : m_raw[1];
-      const float a0 = fast_exp2((m_raw[0] - mn0) * c);
-      const float a1 = fast_exp2((m_raw[1] - mn1) * c);
-      fence_o();
-      // One accumulator block at a time, pinned back into AGPRs: otherwise the
-      // compiler reads all 128 values into VGPRs first.
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][0][r] *= a0;
-        asm volatile("" : "+a"(o[dt][0]));
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][1][r] *= a1;
-        asm volatile("" : "+a"(o[dt][1]));
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        lsum[0][r] *= a0;
-        lsum[1][r] *= a1;
-      }
-      asm volatile("" : "+a"(lsum[0]), "+a"(lsum[1]));
-      m_raw[0] = mn0;
-      m_raw[1] = mn1;
-    }
-  }
-
-  // After a pass that kept every row's first-tile max as m (no per-tile max,
-  // no rescale): whether every row sum is at most 2^64 (so every p was
-  // finite and 1/l is a normal number) and every O^T accumulator finite.
-  // Then the result is the one a running max gives, up to fp32 rounding: m
-  // only sets the exponent range. Reads O, so after fence_o().
-  __device__ __forceinline__ bool sums_in_range() const {
-    float mo = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) mo = max3abs(mo, o[dt][qb][r], o[dt][qb][r + 1]);
-    return lsum[0][0] <= 0x1p64f && lsum[1][0] <= 0x1p64f && mo <= 0x1.fffffep127f;
-  }
-
-  // O (or the range's partial O) of query block qb: O / l, optional padding
-  // correction, bf16, out through the 8 KB staging area `stage` (tile_io.h
-  // row staging, 4 whole 256-byte rows per store); LSE in fp32.
-  template <int qb>
-  __device__ __forceinline__ float finish(float pad_ln, bool pad, bf16* obase, int64_t ors,
-                                          int orow0, int onrows, int lane, bf16* stage) const {
-    const float l_tot = lsum[qb][0];
-    const bool any = l_tot > 0.f;
-    const float lse = any ? (m_raw[qb] * c + __log2f(l_tot)) * kLn2 : -INFINITY;
-    float scale = any ? 1.0f / l_tot : 0.f;
-    if (pad) scale *= 1.0f / (1.0f + expf(pad_ln - lse));
-    const f32x16 ob[4] = {o[0][qb], o[1][qb], o[2][qb], o[3][qb]};
-    stage_acc_rows(ob, scale, lane, stage);
-    stage_rows_out(obase, ors, orow0, onrows, lane, stage);
-    return lse;
   }
 };
 
@@ -634,11 +276,11 @@ __device__ __forceinline__ void fwd_block(const FwdParams& p, int blk, bf16* kv_
     const int b0 = (ntiles - 1) & 1;
     const int kb0 = t0 * kBN;
     if (b0) {
-      w.qk_first<1>();
+      w.qk_first<1>(dma);
       if (kb0 + kBN > it.klen) w.mask<1>(kb0, it.klen);
       w.max_plain<1>();
     } else {
-      w.qk_first<0>();
+      w.qk_first<0>(dma);
       if (kb0 + kBN > it.klen) w.mask<0>(kb0, it.klen);
       w.max_plain<0>();
     }
@@ -661,9 +303,9 @@ __device__ __forceinline__ void fwd_block(const FwdParams& p, int blk, bf16* kv_
       constexpr bool NEXT = decltype(next)::value;
       top(t);
       const int kbn = (t0 + t + 1) * kBN;
-      w.tile<SB, NEXT, TRACK>(stage_addr(t + 1) - stage_addr(t), kbn + kBN > it.klen, kbn, it.klen,
+      w.tile<SB, NEXT, TRACK, false>(stage_addr(t + 1) - stage_addr(t), kbn + kBN > it.klen, kbn, it.klen,
                               dma);
-      if constexpr (NEXT && TRACK) w.update_max();
+      if constexpr (NEXT && TRACK) w.update_max<false>();
     };
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
@@ -966,23 +608,45 @@ static int fwd_scratch(void** out) {
   return AA_OK;
 }
 
-// Which head_dim-128 kernel runs: the two-group kernel of attn_fwd_pp.hip (0)
-// up to kPingPongMaxSk keys, where a work item's fixed costs weigh most, and
-// this file's one-wave-per-SIMD kernel (1) beyond. Measured on MI355X at
-// B = 1-2, 4096 queries: the two-group kernel is 5-8% faster at 512 and 1024
-// keys, the two tie at 2048, the one-wave kernel is ~3% faster at 4096.
-// AA_FWD_KERNEL=pp|1w forces one (tests run both on every shape); -1 for
+// Which head_dim-128 kernel runs.
+//   2, the key-split kernel of attn_fwd_ks.hip (64 queries per workgroup, the
+//      keys split over its waves), where it takes least: problems whose 256-
+//      query items fill a fraction of the chip. Time in us of one round of a
+//      form = kRoundUs + its tiles per wave x kKsTileUs or kTileUs, plus
+//      kMergeUs for the partials' way through memory and the combine launch;
+//      the constants are fits to graph-timed calls on MI355X (16 heads, to
+//      within 10%). Measured against the other two: B=1 256 tokens 10.8 ->
+//      8.8 us, 512 19.8 -> 10.8, 768 20.3 -> 12.7, 1024 22.8 -> 15.3, B=2
+//      1024 31.8 -> 27.6, 1024 x 512 keys 19.4 -> 10.9; where the rule turns
+//      it down: 1280 tokens 29.4 against 27.7, 256 x 4096 keys 30.3 against
+//      23.0, 1024 x 64 keys 8.6 against 6.5.
+//   else up to kPingPongMaxSk keys 0, the two-group kernel of attn_fwd_pp.hip,
+//      which hides more of a work item's fixed costs, and beyond 1, this
+//      file's one-wave-per-SIMD kernel. At B = 1-2, 4096 queries: the
+//      two-group kernel is 5-8% faster at 512 and 1024 keys, the two tie at
+//      2048, the one-wave kernel is ~3% faster at 4096.
+// AA_FWD_KERNEL=pp|1w|ks forces one (tests run them on every shape); -1 for
 // another value.
 constexpr int64_t kPingPongMaxSk = 2048;
-static int fwd_kernel_choice(int64_t Sk) {
+constexpr double kRoundUs = 4.0, kTileUs = 1.78, kKsTileUs = 2.1, kMergeUs = 8.0;
+static int fwd_kernel_choice(int64_t B, const FwdParams& p) {
   const char* e = std::getenv("AA_FWD_KERNEL");
   if (e && *e) {
     const std::string v = e;
     if (v == "pp") return 0;
     if (v == "1w") return 1;
+    if (v == "ks") return 2;
     return -1;
   }
-  return Sk <= kPingPongMaxSk ? 0 : 1;
+  const int64_t ncu = std::max(device_cu_count(), 1), tiles = (p.Sk + kBN - 1) / kBN;
+  const int64_t ks_blocks = B * p.H * ((p.Sq + kKsQueries - 1) / kKsQueries);
+  const double ks = (double)((ks_blocks + ncu - 1) / ncu) *
+                    (kRoundUs + kKsTileUs * (double)((tiles + 3) / 4));
+  double other = (double)((p.full_blocks + ncu - 1) / ncu) * (kRoundUs + kTileUs * (double)tiles);
+  if (p.split_items > 0)
+    other += kRoundUs + kTileUs * (double)((tiles + p.nsplit - 1) / p.nsplit) + kMergeUs;
+  if (ks < other) return 2;
+  return p.Sk <= kPingPongMaxSk ? 0 : 1;
 }
 
 // Which form of the one-wave kernel runs: the first-tile max (true) saves
@@ -1034,8 +698,12 @@ extern "C" int aa_attn_fwd(const aa_attn_fwd_args* a, void* stream) {
   if (a->B == 0 || a->Sq == 0) return AA_OK;
   hipStream_t st = (hipStream_t)stream;
   const int blocks = p.full_blocks + p.split_items * p.nsplit;
-  const int which = fwd_kernel_choice(p.Sk);
-  if (which < 0) return fail(AA_EINVAL, "AA_FWD_KERNEL must be pp or 1w");
+  const int which = fwd_kernel_choice(a->B, p);
+  if (which < 0) return fail(AA_EINVAL, "AA_FWD_KERNEL must be pp, 1w or ks");
+  if (which == 2) {
+    launch_attn_fwd_ks(p, a->B, st);
+    return check_launch("attn_fwd ks");
+  }
   if (which == 0) launch_attn_fwd_pp(p, (unsigned)blocks, st);
   else if (fwd_first_tile_max(p, blocks)) {
     attn_fwd_kernel<false><<<dim3((unsigned)blocks), kWaves * 64, 0, st>>>(p);

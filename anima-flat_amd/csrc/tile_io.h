@@ -148,6 +148,22 @@ __device__ __forceinline__ void dma16_sva(const void* sbase, uint32_t voff, uint
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbu), "s"(m0)
                : "memory", "m0");
 }
+// The same from sbase + voff + kOff to LDS at lds_byte + kLds + 16 lane, with
+// both constants in the instructions: the load's immediate offset (which it
+// adds to the LDS address as well, so M0 is set that much lower) and M0's add,
+// which the compiler would otherwise keep as one register per destination.
+template <int kOff, int kLds>
+__device__ __forceinline__ void dma16_sva_off(const void* sbase, uint32_t voff, uint32_t lds_byte) {
+  static_assert(kOff >= 0 && kOff < 4096, "immediate offset range");
+  const uint32_t base = __builtin_amdgcn_readfirstlane(lds_byte);
+  const uint64_t sb = (uint64_t)(uintptr_t)sbase;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)sb);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(sb >> 32));
+  const uint64_t sbu = ((uint64_t)hi << 32) | (uint64_t)lo;
+  asm volatile("s_add_i32 m0, %2, %4\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(voff),
+               "s"(sbu), "s"(base), "n"(kOff), "n"(kLds - kOff)
+               : "memory", "m0", "scc");
+}
 // The same with the LDS destination as a pointer into __shared__ memory.
 __device__ __forceinline__ void dma16_sv(const void* sbase, uint32_t voff, const void* lds_dst) {
   dma16_sva(sbase, voff, (uint32_t)(uintptr_t)(lds_void*)lds_dst);

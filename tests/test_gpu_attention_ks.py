@@ -1,0 +1,94 @@
+"""GPU parity of the key-split forward (one workgroup per 64 queries, the keys
+split over its four waves and merged in LDS) against the CPU oracle, at the
+edges of its tiles: query blocks of 64, key tiles of 64 dealt to 4 waves, tiles
+moved back to end at the key length, waves without keys."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from conftest import parity
+from oracle import attn_oracle as ref
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+# LSE: the log of a sum of fp32 probabilities. Relative errors of the sum: its
+# exp2 arguments s c - m c (2^-24 of up to ~300) and the device's exp2 and log2
+# (1 ulp each), together below 5e-5.
+LSE_TOL = {"max_abs": 1e-4, "rel_l2": 1e-5}
+
+
+def _inputs(B, Sq, Sk, H, seed):
+    g = torch.Generator().manual_seed(seed)
+    return [ref.bf16_normal(s, g) for s in ((B, Sq, H, 128), (B, Sk, H, 128), (B, Sk, H, 128))]
+
+
+@pytest.mark.parametrize(
+    "B,Sq,Sk,H,lens",
+    [
+        (1, 1, 1, 1, None),
+        (1, 63, 64, 2, None),  # one key tile: three waves hold no keys
+        (2, 64, 65, 3, None),  # two tiles, the second moved back over 63 keys
+        (1, 65, 255, 2, None),  # every wave one tile, the last partial
+        (1, 100, 256, 1, None),
+        (1, 129, 257, 2, None),  # a second round of tiles for wave 0 only
+        (2, 70, 513, 2, [513, 1]),  # one key
+        (3, 33, 300, 2, [63, 64, 192]),  # shorter than a tile, whole tiles
+        (1, 300, 1000, 8, None),
+        (1, 128, 4100, 2, None),  # many tiles per wave (lazy rescale)
+    ],
+)
+def test_key_split_forward(pkg, monkeypatch, B, Sq, Sk, H, lens):
+    q, k, v = _inputs(B, Sq, Sk, H, 100 + Sq + Sk)
+    seq = torch.tensor(lens if lens is not None else [Sk] * B, dtype=torch.int32)
+    kd, vd = k.to("cuda", BF), v.to("cuda", BF)
+    for b, n in enumerate(seq.tolist()):  # rows past a key length hold anything
+        kd[b, n:] = float("nan")
+        vd[b, n:] = float("inf")
+    monkeypatch.setenv("AA_FWD_KERNEL", "ks")
+    qd = q.to("cuda", BF)
+    if lens is None:
+        out, lse = torch.ops.anima_flat.fa_fwd(qd, kd, vd)
+    else:
+        out, lse = torch.ops.anima_flat.fa_fwd_k(qd, kd, vd, seq.to("cuda"))
+    pad = torch.log((Sk + 5 - seq).float())
+    fused = pkg.cross_attention_trimmed(qd, kd, vd, seq.to("cuda"), pad.to("cuda"))
+    torch.cuda.synchronize()
+    eo, el = ref.attention_lse(q, k, v, seq)
+    parity(out, eo, name="out")
+    if lens is None:  # the instance that leaves the LSE out
+        assert torch.equal(torch.ops.anima_flat.fa_fwd_nolse(qd, kd, vd), out)
+    parity(lse, el, **LSE_TOL, name="lse")
+    parity(fused.view(B, Sq, H, 128), ref.cross_attention_trimmed(q, k, v, seq, pad), name="fused")
+
+
+def test_key_split_strides_and_route(pkg, monkeypatch):
+    """The default rule takes it for 512 queries of 16 heads, with the same bits as when
+    forced, and it reads strided views (v inside a fused projection) in place."""
+    g = torch.Generator().manual_seed(7)
+    qkv = ref.bf16_normal((1, 512, 3, 16, 128), g).to("cuda", BF)
+    q, k, v = (qkv[:, :, i] for i in range(3))
+    a = pkg.attention(q, k, v)
+    monkeypatch.setenv("AA_FWD_KERNEL", "ks")
+    b = pkg.attention(q, k, v)
+    assert torch.equal(a, b)
+    e = ref.attention_sdpa(*(t.float().cpu() for t in (q, k, v)))
+    parity(a.view(1, 512, 16, 128), e, name="strided")
+
+
+def test_key_split_growing_scores(pkg, monkeypatch):
+    """Scores that grow along the keys by ~28 log2 units per tile: every wave raises its
+    maximum at each of its tiles, and most of the waves' partial results weigh nothing."""
+    g = torch.Generator().manual_seed(8)
+    q, k, v = _inputs(1, 64, 700, 1, 9)
+    u = torch.randn(128, generator=g)
+    u = u / u.norm()
+    q = (q + 60.0 * u).to(BF).float()
+    k = (k + torch.linspace(0.0, 40.0, 700)[None, :, None, None] * u).to(BF).float()
+    monkeypatch.setenv("AA_FWD_KERNEL", "ks")
+    out, lse = torch.ops.anima_flat.fa_fwd(*(t.to("cuda", BF) for t in (q, k, v)))
+    eo, el = ref.attention_lse(q, k, v, None)
+    parity(out, eo, name="out")
+    parity(lse, el, **LSE_TOL, name="lse")
