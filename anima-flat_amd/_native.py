@@ -1,0 +1,62 @@
+"""Native dispatcher kernels of the package's torch ops (csrc/torch_ops.cpp).
+
+`attach(qualname, impl)` gives a registered op CUDA and AutogradCUDA kernels
+that call libanima_attn.so straight from C++; `impl`, the op's Python function,
+stays the kernel of every other dispatch key and takes the calls the native
+kernels hand back (copies, other dtypes, errors). The extension is built with
+the library (build.py); without it the ops run the same HIP kernels through
+Python, which is reported once.
+"""
+
+from __future__ import annotations
+
+import importlib.util
+import warnings
+from pathlib import Path
+
+import torch  # noqa: F401  (the extension binds to torch's libraries)
+
+from . import _lib
+
+EXT_PATH = Path(__file__).resolve().with_name("_anima_torch.so")
+
+NATIVE_OPS = frozenset({
+    "anima_flat::fa_fwd", "anima_flat::fa_fwd_nolse", "anima_flat::fa_fwd_k", "anima_flat::fa_bwd",
+    "anima_flat_amd::fa_fwd_k_ctx", "anima_flat_amd::attend_d384",
+    "anima_flat::qkv_norm_rope", "anima_flat::qkv_norm_rope_v", "anima_flat::qkv_norm_rope_bwd",
+    "anima_flat::head_norm", "anima_flat::head_norm_bwd",
+    "anima_flat_amd::qkv_proj_norm_rope", "anima_flat_amd::proj_head_norm",
+    "anima_flat_amd::kv_proj_norm",
+})
+
+_ext = None
+_missing = False
+
+
+def _load():
+    """The extension module, or None (reported once) when it is not built."""
+    global _ext, _missing
+    if _ext is None and not _missing:
+        if not (EXT_PATH.exists() and _lib.LIB_PATH.exists()):
+            _missing = True
+            if _lib.LIB_PATH.exists():
+                warnings.warn(
+                    f"{EXT_PATH.name} is not built (run `python anima-flat_amd/build.py`): "
+                    "every op call goes through Python", RuntimeWarning, stacklevel=3)
+            return None
+        spec = importlib.util.spec_from_file_location("_anima_torch", EXT_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        if module.abi_version() != _lib.ABI_VERSION:
+            raise RuntimeError(
+                f"{EXT_PATH.name} is linked to ABI version {module.abi_version()}, expected {_lib.ABI_VERSION}")
+        _ext = module
+    return _ext
+
+
+def attach(qualname: str, impl) -> None:
+    """Give op `qualname` its native kernels, if it has any."""
+    if qualname in NATIVE_OPS:
+        ext = _load()
+        if ext is not None:
+            ext.attach(qualname, impl)

@@ -1,9 +1,10 @@
-"""Builds libanima_attn.so from csrc/*.hip with hipcc for gfx950.
+"""Builds libanima_attn.so from csrc/*.hip with hipcc for gfx950, and the torch
+extension _anima_torch.so (csrc/torch_ops.cpp, host code only) with g++.
 
-Objects go to `_build/` next to this file and the library to
-`libanima_attn.so` in this directory, where `_lib.py` loads it from. Every
-source compiles in parallel; nothing is cached between calls (the caller asks
-for a build, so it gets one).
+Objects go to `_build/` next to this file and the libraries to this directory,
+where `_lib.py` and `_native.py` load them from. Every source compiles in
+parallel; nothing is cached between calls (the caller asks for a build, so it
+gets one).
 
 Run as a script to build: ``python anima-flat_amd/build.py``.
 """
@@ -14,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -31,6 +33,11 @@ ARCH = "gfx950"
 # that the attention library holds only the path's entry points.
 CALIB_SOURCE = "calib_mfma.hip"
 CALIB_LIB_PATH = HERE / "libanima_calib.so"
+
+# The torch ops' native dispatcher kernels: host code against torch's headers,
+# linked to the attention library beside it.
+TORCH_SOURCE = "torch_ops.cpp"
+TORCH_LIB_PATH = HERE / "_anima_torch.so"
 
 # Packed fp32 VALU forms are disabled for all device code: the compiler then
 # emits only scalar v_fma_f32/v_mul_f32 for float arithmetic.
@@ -116,9 +123,30 @@ def _run(cmd: list[str]) -> None:
         _check_resources(proc.stderr, cmd[cmd.index("-c") + 1])
 
 
+def _torch_commands() -> tuple[list[str], list[str]]:
+    """The compile and link commands of the torch extension."""
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    obj = str(BUILD / (Path(TORCH_SOURCE).stem + ".o"))
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    compile_cmd = [
+        "g++", "-O2", "-std=c++17", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{rocm}/include",
+        f"-I{sysconfig.get_path('include')}", "-c", str(CSRC / TORCH_SOURCE), "-o", obj,
+    ]
+    link_cmd = [
+        "g++", "-shared", "-fPIC", "-o", str(TORCH_LIB_PATH) + ".tmp", obj, f"-L{root}/lib", f"-L{HERE}",
+        "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lc10", "-lc10_hip", "-lanima_attn",
+        "-Wl,-rpath,$ORIGIN",
+    ]
+    return compile_cmd, link_cmd
+
+
 def build(verbose: bool = False) -> Path:
-    """Compile every source, link libanima_attn.so and the calibration library
-    libanima_calib.so; returns the attention library's path."""
+    """Compile every source, link libanima_attn.so, the calibration library
+    libanima_calib.so and the torch extension; returns the attention library's path."""
     cc = hipcc()
     SGPR_SPILL_WARNINGS.clear()
     BUILD.mkdir(exist_ok=True)
@@ -130,6 +158,8 @@ def build(verbose: bool = False) -> Path:
             objs.append(str(obj))
         cmds.append([cc, *DEVICE_FLAGS, *SOURCE_FLAGS.get(src, []), RESOURCE_REMARK, "-c",
                      str(CSRC / src), "-o", str(obj)])
+    torch_compile, torch_link = _torch_commands()
+    cmds.append(torch_compile)
     workers = max(1, min(len(cmds), os.cpu_count() or 1, 8))
     with ThreadPoolExecutor(workers) as pool:
         for cmd, _ in zip(cmds, pool.map(_run, cmds)):
@@ -145,6 +175,8 @@ def build(verbose: bool = False) -> Path:
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(ctmp),
           str(BUILD / (Path(CALIB_SOURCE).stem + ".o"))])
     os.replace(ctmp, CALIB_LIB_PATH)
+    _run(torch_link)
+    os.replace(str(TORCH_LIB_PATH) + ".tmp", TORCH_LIB_PATH)
     return LIB_PATH
 
 

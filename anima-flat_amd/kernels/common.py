@@ -16,6 +16,8 @@ from __future__ import annotations
 
 import torch
 
+from .. import _native
+
 
 def _check(*ts: torch.Tensor) -> None:
     for t in ts:
@@ -30,11 +32,18 @@ def is_registered(qualname: str) -> bool:
 
 
 def custom_op(qualname: str, **kwargs):
-    """torch.library.custom_op(qualname, **kwargs), refusing an existing name."""
+    """torch.library.custom_op(qualname, **kwargs), refusing an existing name; the op
+    gets its native dispatcher kernels, where it has them (_native.attach)."""
     if is_registered(qualname):
         raise RuntimeError(
             f"torch op {qualname} is already registered in this process (most likely by "
             "anima-flat's own module of the same name); import either that module or "
             "anima_flat_amd's, not both"
         )
-    return torch.library.custom_op(qualname, **kwargs)
+
+    def register(fn):
+        op = torch.library.custom_op(qualname, **kwargs)(fn)
+        _native.attach(qualname, fn)
+        return op
+
+    return register

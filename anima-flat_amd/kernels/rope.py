@@ -42,6 +42,9 @@ def _launch_qkv(qkv, q_weight, k_weight, cos, sin, heads, eps, with_v):
     q = qkv.new_empty((B, S, heads, hd))
     k = torch.empty_like(q)
     v = torch.empty_like(q) if with_v else None
+    # Held to the launch: a converted copy freed before the next one is made
+    # would hand it its memory.
+    qw, kw, c32, s32 = _f32(q_weight), _f32(k_weight), _f32(cos), _f32(sin)
     with torch.cuda.device(qkv.device):
         _lib.check(
             _lib.lib().aa_qkv_norm_rope_fwd(
@@ -49,10 +52,10 @@ def _launch_qkv(qkv, q_weight, k_weight, cos, sin, heads, eps, with_v):
                 q.data_ptr(),
                 k.data_ptr(),
                 _lib.ptr(v),
-                _f32(q_weight).data_ptr(),
-                _f32(k_weight).data_ptr(),
-                _f32(cos).data_ptr(),
-                _f32(sin).data_ptr(),
+                qw.data_ptr(),
+                kw.data_ptr(),
+                c32.data_ptr(),
+                s32.data_ptr(),
                 B,
                 S,
                 heads,
@@ -221,6 +224,7 @@ def _qkv_norm_rope_bwd(qkv, dq, dk, dv, q_weight, k_weight, cos, sin, heads, eps
     dkw = torch.empty(hd, dtype=torch.float32, device=qkv.device)
     ws_bytes = _lib.lib().aa_qkv_norm_rope_bwd_workspace(B, S, heads, hd)
     ws = torch.empty(max(ws_bytes // 4, 1), dtype=torch.float32, device=qkv.device)
+    qw, kw, c32, s32 = _f32(q_weight), _f32(k_weight), _f32(cos), _f32(sin)  # held to the launch
     with torch.cuda.device(qkv.device):
         _lib.check(
             _lib.lib().aa_qkv_norm_rope_bwd(
@@ -229,10 +233,10 @@ def _qkv_norm_rope_bwd(qkv, dq, dk, dv, q_weight, k_weight, cos, sin, heads, eps
                 dk.data_ptr(),
                 dv.data_ptr(),
                 dqkv.data_ptr(),
-                _f32(q_weight).data_ptr(),
-                _f32(k_weight).data_ptr(),
-                _f32(cos).data_ptr(),
-                _f32(sin).data_ptr(),
+                qw.data_ptr(),
+                kw.data_ptr(),
+                c32.data_ptr(),
+                s32.data_ptr(),
                 dqw.data_ptr(),
                 dkw.data_ptr(),
                 ws.data_ptr(),

@@ -1,0 +1,116 @@
+"""The ops' native dispatcher kernels against their Python functions: the same
+results, autograd behaviour and errors, whichever of the two a call reaches."""
+
+from __future__ import annotations
+
+import importlib
+
+import pytest
+import torch
+
+from oracle import attn_oracle as ref
+
+BF = torch.bfloat16
+
+
+def _qkv(device="cuda", Sq=70, Sk=90, H=2):
+    g = torch.Generator().manual_seed(3)
+    return [ref.bf16_normal((1, s, H, 128), g).to(device, BF) for s in (Sq, Sk, Sk)]
+
+
+def _fake_forward(pkg):
+    q, k, v = (torch.empty(2, s, 3, 128, dtype=BF, device="cuda", requires_grad=True) for s in (5, 7, 7))
+    out = pkg.attention(q, k, v)
+    assert out.shape == (2, 5, 384) and out.device.type == "cuda" and out.requires_grad
+    return out, (q, k, v)
+
+
+def test_fake_forward(pkg):
+    """Fake CUDA tensors reach the fake implementations through the native autograd kernels
+    (no GPU is touched)."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode():
+        _fake_forward(pkg)
+
+
+@pytest.mark.gpu
+def test_fake_backward(pkg):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode():
+        out, leaves = _fake_forward(pkg)
+        grads = torch.autograd.grad(out, leaves, torch.empty_like(out))
+        assert [g.shape for g in grads] == [t.shape for t in leaves]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["plain", "head_major", "misaligned", "last_dim_strided"])
+def test_same_result_from_both_paths(pkg, form):
+    """Views the native kernel reads in place and views that go to the Python function (which
+    copies them) give the bits of a plain call."""
+    q, k, v = _qkv()
+    if form == "head_major":
+        kx = k.transpose(1, 2).contiguous().transpose(1, 2)
+    elif form == "misaligned":
+        kx = torch.empty(k.numel() + 4, dtype=BF, device="cuda")[4:].view(k.shape).copy_(k)
+    elif form == "last_dim_strided":
+        kx = torch.stack((k, k), -1)[..., 0]
+    else:
+        kx = k.clone()
+    want = torch.ops.anima_flat.fa_fwd(q, k, v)
+    got = torch.ops.anima_flat.fa_fwd(q, kx, v)
+    direct = importlib.import_module("anima_flat_amd.attention")._launch_fwd(q, kx, v, want_lse=True)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+    assert all(torch.equal(a, b) for a, b in zip(want, direct))
+
+
+@pytest.mark.gpu
+def test_autograd_behaviour(pkg):
+    """Saved tensors pass the saved-tensor hooks, a second backward needs retain_graph, ops
+    without a backward raise on it and not before, and so does a double backward."""
+    leaves = [t.requires_grad_(True) for t in _qkv()]
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(tuple(t.shape)), t.clone())[1], lambda t: t):
+        out = pkg.attention(*leaves)
+    assert len(seen) == 5  # q, k, v, out, lse
+    grads = torch.autograd.grad(out.float().pow(2).sum(), leaves, retain_graph=True)
+    again = torch.autograd.grad(out.float().pow(2).sum(), leaves)
+    assert all(torch.equal(a, b) for a, b in zip(grads, again))
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out.float().pow(2).sum(), leaves)
+
+    nolse = torch.ops.anima_flat.fa_fwd_nolse(*leaves)
+    assert nolse.requires_grad
+    with pytest.raises(RuntimeError, match="fa_fwd_nolse.default but no autograd formula"):
+        nolse.sum().backward()
+
+    first = torch.autograd.grad(pkg.attention(*leaves).float().pow(2).sum(), leaves, create_graph=True)
+    with pytest.raises(RuntimeError, match="fa_bwd.default but no autograd formula"):
+        torch.autograd.grad(first[0].float().sum(), leaves)
+
+
+@pytest.mark.gpu
+def test_errors_are_the_python_functions(pkg):
+    q, k, v = _qkv()
+    with pytest.raises(ValueError, match="only bfloat16"):
+        torch.ops.anima_flat.fa_fwd(q.half(), k.half(), v.half())
+    with pytest.raises(ValueError, match="same shape"):
+        torch.ops.anima_flat.fa_fwd(q, k, v[:, :5])
+    with pytest.raises(ValueError, match="seqused_k must be"):
+        torch.ops.anima_flat.fa_fwd_k(q, k, v, torch.ones(2, dtype=torch.int32, device="cuda"))
+    with pytest.raises(ValueError, match="CUDA tensors required"):
+        pkg.attention(q.cpu(), k.cpu(), v.cpu())
+
+
+@pytest.mark.gpu
+def test_weights_in_another_dtype(pkg):
+    """bf16 norm weights and tables are converted, each to a tensor of its own that lives
+    until the launch."""
+    g = torch.Generator().manual_seed(4)
+    qkv = ref.bf16_normal((1, 40, 3 * 256), g).to("cuda", BF)
+    qw, kw = (ref.bf16_normal((128,), g).cuda() for _ in range(2))
+    cos, sin = (ref.bf16_normal((40, 64), g).cuda() for _ in range(2))
+    want = pkg.qkv_norm_rope(qkv, qw, kw, cos, sin, 2, 1e-6)
+    got = pkg.qkv_norm_rope(qkv, *(t.to(BF) for t in (qw, kw, cos, sin)), 2, 1e-6)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
