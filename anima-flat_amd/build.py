@@ -26,7 +26,8 @@ LIB_NAME = "libanima_attn.so"
 LIB_PATH = HERE / LIB_NAME
 SOURCES = (
     "abi.hip", "prologue.hip", "ctx_scale.hip", "context.hip", "rowquant.hip", "attn_fwd.hip",
-    "attn_fwd_pp.hip", "attn_fwd_ks.hip", "attn_fwd_d384.hip", "attn_bwd.hip", "attn_bwd_dkdv.hip", "qkv_proj.hip",
+    "attn_fwd_pp.hip", "attn_fwd_ks.hip", "attn_fwd_d384.hip", "attn_bwd.hip", "attn_bwd_dq_ks.hip",
+    "attn_bwd_dkdv.hip", "qkv_proj.hip",
 )
 ARCH = "gfx950"
 # The measurement's MFMA-rate calibration (bench.py), a library of its own so
@@ -55,7 +56,8 @@ DEVICE_FLAGS = [
 
 RESOURCE_REMARK = "-Rpass-analysis=kernel-resource-usage"
 
-# Per-source extra flags. attn_fwd.hip, attn_fwd_ks.hip and attn_bwd_dkdv.hip run one wave per
+# Per-source extra flags. attn_fwd.hip, attn_fwd_ks.hip, attn_bwd_dq_ks.hip
+# and attn_bwd_dkdv.hip run one wave per
 # SIMD, where the compiler would otherwise give every MFMA accumulator the
 # AGPR file; their score accumulators must be VGPRs (the VALU reads them), so
 # the builtin MFMAs are compiled in the VGPR form and the output accumulators
@@ -63,6 +65,7 @@ RESOURCE_REMARK = "-Rpass-analysis=kernel-resource-usage"
 SOURCE_FLAGS: dict[str, list[str]] = {
     "attn_fwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attn_fwd_ks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "attn_bwd_dq_ks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attn_bwd_dkdv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 

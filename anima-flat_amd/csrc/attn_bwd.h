@@ -31,20 +31,40 @@ struct Params {
   bf16* dv;
   int64_t s_do[3], s_q[3], s_k[3], s_v[3], s_o[3], s_dq[3], s_dk[3], s_dv[3];
   float* stats;  // [B][H][ntq][kStat]
-  // Query split of the dK/dV kernels (see dkdv_split): with nsplit > 1,
-  // workgroup (split, b, h, key block) covers query tiles split * ceil(ntq /
-  // nsplit) .. and writes its fp32 dV^T / dK^T accumulators to part (layout
-  // above), which the combine pass sums in a fixed order.
+  // Query split of the dK/dV kernels (see dkdv_split): items (key blocks) from
+  // full_items on are split, workgroup full_items + j covering query tiles
+  // split * ceil(ntq / nsplit) .. (split = j / split_items) of item full_items
+  // + j % split_items; its fp32 dV^T / dK^T accumulators go to record j of
+  // part (layout above), which the combine pass sums in a fixed order.
   float* part;
-  int nsplit;
+  int nsplit, full_items, split_items;
   int H, Sq, Sk, ntq, ntk;
   float c;      // scale * log2(e)
   float scale;  // softmax scale
 };
 
+// Workgroup `block` of a dK/dV kernel -> item (b, h, key block), its query
+// split and partial record (-1: unsplit). XCD-aware within each part.
+__device__ __forceinline__ void dkdv_item(const Params& p, int block, int& item, int& split, int& rec) {
+  split = 0;
+  rec = -1;
+  if (block < p.full_items) {
+    item = xcd_remap(block, p.full_items);
+    return;
+  }
+  rec = xcd_remap(block - p.full_items, p.split_items * p.nsplit);
+  split = rec / p.split_items;
+  item = p.full_items + rec - split * p.split_items;
+}
+
 // Launches the one-wave-per-SIMD dK/dV kernel of attn_bwd_dkdv.hip over
-// `total` workgroups (nkblk key blocks per (batch, head), times nsplit).
+// `total` workgroups (nkblk key blocks per (batch, head)).
 void launch_dkdv1w(const Params& p, int nkblk, int total, hipStream_t stream);
+
+// Launches the key-split dQ kernel of attn_bwd_dq_ks.hip over `items` of
+// dq_kernel's items (256 queries of one (batch, head); nqitem per (batch,
+// head)) from first_item on.
+void launch_dq_ks(const Params& p, int first_item, int items, int nqitem, hipStream_t stream);
 
 }  // namespace bwd
 }  // namespace aa

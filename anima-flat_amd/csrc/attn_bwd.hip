@@ -75,17 +75,15 @@ constexpr int kDkQueue = 8;   // A operands in flight per wave
 constexpr int kDkStages = 4;  // query tiles in the LDS ring
 
 __global__ __launch_bounds__(kDkWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void dkdv_kernel(Params p, int nkblk, int total_blocks) {
+void dkdv_kernel(Params p, int nkblk) {
   __shared__ __attribute__((aligned(1024))) bf16 rows[kDkStages][2][kTileElems];  // [stage][Q, dO]
   __shared__ __attribute__((aligned(1024))) float stat[kDkStages][kStat];
   __shared__ __attribute__((aligned(1024))) bf16x8 pslot[4][4][64];  // [pair][c4][lane]
 
-  const int logical = xcd_remap(blockIdx.x, total_blocks);
-  const int per_split = total_blocks / p.nsplit;
-  const int split = logical / per_split;
-  const int rest = logical - split * per_split;
-  const int kblk = rest % nkblk;
-  const int bh = rest / nkblk;
+  int item, split, rec;
+  dkdv_item(p, blockIdx.x, item, split, rec);
+  const int kblk = item % nkblk;
+  const int bh = item / nkblk;
   const int b = bh / p.H, h = bh - (bh / p.H) * p.H;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -108,7 +106,7 @@ void dkdv_kernel(Params p, int nkblk, int total_blocks) {
   const bf16* qbase = p.q + b * p.s_q[0] + h * p.s_q[2];
   const bf16* dobase = p.dout + b * p.s_do[0] + h * p.s_do[2];
   // Query tiles tq0 .. tq0 + ntiles - 1 (all of them without a split).
-  const int tper = (p.ntq + p.nsplit - 1) / p.nsplit;
+  const int tper = rec < 0 ? p.ntq : (p.ntq + p.nsplit - 1) / p.nsplit;
   const int tq0 = min(split * tper, p.ntq);
   const int ntiles = min(tper, p.ntq - tq0);
   const float* statb = p.stats + ((int64_t)bh * p.ntq + tq0) * kStat;
@@ -268,10 +266,10 @@ void dkdv_kernel(Params p, int nkblk, int total_blocks) {
   // dV (A) / dK (B) rows out through LDS staging: the stages of tiles
   // ntiles-4 and ntiles-3 are free (B may still be reading tile ntiles-1 in
   // its final M block; no DMA is in flight).
-  if (p.nsplit > 1) {
+  if (rec >= 0) {
     // Partial accumulators, 16 coalesced 1 KB stores per wave: float4 j of
     // lane l at ((logical * 8 + wave) * 16 + j) * 64 + l.
-    f32x4* dst = reinterpret_cast<f32x4*>(p.part) + ((int64_t)logical * kDkWaves + wave) * 16 * 64 + lane;
+    f32x4* dst = reinterpret_cast<f32x4*>(p.part) + ((int64_t)rec * kDkWaves + wave) * 16 * 64 + lane;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const f32x4 v4 = {acc[j >> 2][4 * (j & 3)], acc[j >> 2][4 * (j & 3) + 1], acc[j >> 2][4 * (j & 3) + 2],
@@ -298,14 +296,15 @@ void dkdv_kernel(Params p, int nkblk, int total_blocks) {
 // and one 16-byte store (8-byte stores of one lane's half took 11.7 us for
 // B=2, 512 keys, 16 heads, 2 splits).
 constexpr int kMaxDkSplit = 4;
-__global__ __launch_bounds__(256) void dkdv_combine_kernel(Params p, int nkblk, int per_split) {
+__global__ __launch_bounds__(256) void dkdv_combine_kernel(Params p, int nkblk) {
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (rest, wave, j, li)
   const int li = (int)(gid & 31);
   const int j = (int)((gid >> 5) & 15);
   const int wave = (int)((gid >> 9) & 7);
   const int rest = (int)(gid >> 12);
+  const int per_split = p.split_items;
   if (rest >= per_split) return;
-  const int kblk = rest % nkblk, bh = rest / nkblk;
+  const int item = p.full_items + rest, kblk = item % nkblk, bh = item / nkblk;
   const int b = bh / p.H, h = bh - b * p.H;
   const int key = kblk * kKeysPerWg + (wave & 3) * 32 + li;
   if (key >= p.Sk) return;
@@ -577,33 +576,43 @@ static bool stride_ok(const int64_t* s) {
          s[1] < (1ll << 40) && s[2] < (1ll << 40);
 }
 
-// Query splits of dkdv_kernel: when its workgroups (one per 128 keys of each
-// (batch, head)) fill at most half of the CUs, as for the 512-key text
-// context at B = 2 and 16 heads (128 workgroups), each key block's query
-// tiles are split over up to 4 workgroups, each covering at least 4 tiles.
-static int dkdv_split(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int ncu) {
-  const int64_t blocks = B * H * ((Sk + kKeysPerWg - 1) / kKeysPerWg);
+// Query splits of the dK/dV kernels. Their items (128 keys of one (batch,
+// head)) run in rounds of one per CU; when the items of a partial last round
+// fill at most half of the CUs, as the 128 items of the 512-key text context
+// at B = 2 and 16 heads or the last 32 of 2304 tokens' 288, each of them is
+// split over up to 4 workgroups of at least 4 query tiles. Behind whole
+// rounds the split has to save kDkTailTiles tiles, what the partials and the
+// combine pass cost (~14 us): 2304 tokens 188 -> 163 us for the backward, 2560
+// 210 -> 192.
+constexpr int kDkTailTiles = 8;
+struct DkSplit {
+  int full_items, split_items, nsplit;
+};
+static DkSplit dkdv_split(int64_t B, int64_t Sq, int64_t Sk, int64_t H, int ncu) {
+  const int64_t items = B * H * ((Sk + kKeysPerWg - 1) / kKeysPerWg);
   const int64_t ntq = (Sq + kT - 1) / kT;
-  if (ncu <= 0 || blocks <= 0 || 2 * blocks > ncu) return 1;
-  int64_t ns = std::min<int64_t>(kMaxDkSplit, ncu / blocks);
-  ns = std::min<int64_t>(ns, ntq / 4);
-  return (int)std::max<int64_t>(ns, 1);
+  const DkSplit whole{(int)items, 0, 1};
+  if (ncu <= 0 || items <= 0) return whole;
+  const int64_t rem = items % ncu;
+  if (rem == 0 || 2 * rem > ncu) return whole;
+  const int64_t ns = std::min<int64_t>(std::min<int64_t>(kMaxDkSplit, ncu / rem), ntq / 4);
+  if (ns < 2 || (items > rem && ntq - (ntq + ns - 1) / ns < kDkTailTiles)) return whole;
+  return DkSplit{(int)(items - rem), (int)rem, (int)ns};
 }
 
 struct WsLayout {
   size_t stats, part, total;
-  int nsplit;
+  DkSplit split;
 };
 
 static WsLayout ws_layout(int64_t B, int64_t Sq, int64_t Sk, int64_t H) {
   const int64_t ntq = (Sq + kT - 1) / kT;
   WsLayout w;
-  w.nsplit = dkdv_split(B, Sq, Sk, H, device_cu_count());
+  w.split = dkdv_split(B, Sq, Sk, H, device_cu_count());
   w.stats = 0;
   w.part = w.stats + (size_t)(B * H * ntq) * kStat * sizeof(float);
-  const int64_t blocks = B * H * ((Sk + kKeysPerWg - 1) / kKeysPerWg);
-  const size_t part_bytes =
-      w.nsplit > 1 ? (size_t)w.nsplit * blocks * kDkParts * 64 * 64 * sizeof(float) : 0;
+  const size_t part_bytes = (size_t)w.split.split_items * (w.split.split_items ? w.split.nsplit : 0) *
+                            kDkParts * 64 * 64 * sizeof(float);
   w.total = w.part + part_bytes;
   return w;
 }
@@ -620,6 +629,32 @@ static int dkdv_kernel_choice() {
     return -1;
   }
   return 1;
+}
+
+// How many of the dQ items (256 queries of one (batch, head)) go to the key-
+// split kernel of attn_bwd_dq_ks.hip, 64 queries per workgroup, instead of
+// dq_kernel: none, the last ones that dq_kernel would run as a partial round,
+// or all (a call of less than one round). Estimated time in us of a round of
+// each is a constant plus its 64-key tiles; the constants are fits to
+// graph-timed calls on MI355X (16 heads). The whole backward, dq_kernel ->
+// key split: B=1 256 tokens 27.3 -> 20.5, 512 45.5 -> 34.0, 1024 70.9 ->
+// 54.6, 2048 128.5 -> 122, 512 x 4096 keys 147 -> 87; where the rule turns it
+// down: 2304 tokens 190 against 202, B=2 1024 x 512 keys 61.8 against 63.2.
+// AA_DQ_KERNEL=2g|ks forces none or all; -1 for another value.
+constexpr double kDqRoundUs = 7.5, kDqTileUs = 1.9, kDqKsRoundUs = 4.3, kDqKsTileUs = 3.6;
+static int64_t dq_ks_items(int64_t items, int64_t Sk) {
+  const char* e = std::getenv("AA_DQ_KERNEL");
+  if (e && *e) {
+    const std::string v = e;
+    if (v == "2g") return 0;
+    if (v == "ks") return items;
+    return -1;
+  }
+  const int64_t ncu = std::max(device_cu_count(), 1), rem = items % ncu, tiles = (Sk + kT - 1) / kT;
+  const double whole = kDqRoundUs + kDqTileUs * (double)tiles;
+  const double split = (double)((4 * rem + ncu - 1) / ncu) *
+                       (kDqKsRoundUs + kDqKsTileUs * (double)((tiles + 3) / 4));
+  return split < whole ? rem : 0;
 }
 
 }  // namespace bwd
@@ -662,6 +697,10 @@ extern "C" int aa_attn_bwd(const aa_attn_bwd_args* a, void* workspace, size_t wo
   if (!(a->softmax_scale > 0.f)) return fail(AA_EINVAL, "attn_bwd: softmax_scale must be > 0");
   const int dkdv_which = bwd::dkdv_kernel_choice();
   if (dkdv_which < 0) return fail(AA_EINVAL, "AA_DKDV_KERNEL must be 1w or 2role");
+  const int64_t nqitem = (a->Sq + bwd::kQueriesPerWg - 1) / bwd::kQueriesPerWg;
+  const int64_t dq_items = a->B * a->H * nqitem;
+  const int64_t dq_ks = bwd::dq_ks_items(dq_items, a->Sk);
+  if (dq_ks < 0) return fail(AA_EINVAL, "AA_DQ_KERNEL must be 2g or ks");
   const bwd::WsLayout wl = bwd::ws_layout(a->B, a->Sq, a->Sk, a->H);
   const size_t need = aa_attn_bwd_workspace(a->B, a->Sq, a->Sk, a->H, a->hd);
   if (need > 0 && (!workspace || workspace_bytes < need))
@@ -692,7 +731,9 @@ extern "C" int aa_attn_bwd(const aa_attn_bwd_args* a, void* workspace, size_t wo
   char* ws = (char*)workspace;
   p.stats = (float*)(ws + wl.stats);
   p.part = (float*)(ws + wl.part);
-  p.nsplit = wl.nsplit;
+  p.nsplit = wl.split.nsplit;
+  p.full_items = wl.split.full_items;
+  p.split_items = wl.split.split_items;
   p.H = (int)a->H;
   p.Sq = (int)a->Sq;
   p.Sk = (int)a->Sk;
@@ -702,25 +743,25 @@ extern "C" int aa_attn_bwd(const aa_attn_bwd_args* a, void* workspace, size_t wo
   p.c = a->softmax_scale * kLog2e;
   hipStream_t st = (hipStream_t)stream;
 
-  const int64_t BH = a->B * a->H;
-  // dq_kernel first: it writes the stats records that dkdv_kernel reads.
+  // dQ first: its kernels write the stats records that the dK/dV kernel reads.
   // Nothing reads the workspace when Sq == 0 (dK = dV = 0 and no dQ rows).
-  if (a->Sq > 0) {
-    const int nqblk = (int)((a->Sq + bwd::kQueriesPerWg - 1) / bwd::kQueriesPerWg);
-    const int total = (int)(BH * nqblk);
-    bwd::dq_kernel<<<dim3((unsigned)total), bwd::kDqWaves * 64, 0, st>>>(p, nqblk, total);
+  if (const int whole = (int)(dq_items - dq_ks)) {
+    bwd::dq_kernel<<<dim3((unsigned)whole), bwd::kDqWaves * 64, 0, st>>>(p, (int)nqitem, whole);
     if (int rc = check_launch("attn_bwd dq")) return rc;
+  }
+  if (dq_ks > 0) {
+    bwd::launch_dq_ks(p, (int)(dq_items - dq_ks), (int)dq_ks, (int)nqitem, st);
+    if (int rc = check_launch("attn_bwd dq ks")) return rc;
   }
   if (a->Sk > 0) {
     const int nkblk = (int)((a->Sk + bwd::kKeysPerWg - 1) / bwd::kKeysPerWg);
-    const int per_split = (int)(BH * nkblk);
-    const int total = per_split * p.nsplit;
+    const int total = p.full_items + p.split_items * p.nsplit;
     if (dkdv_which == 1) bwd::launch_dkdv1w(p, nkblk, total, st);
-    else bwd::dkdv_kernel<<<dim3((unsigned)total), bwd::kDkWaves * 64, 0, st>>>(p, nkblk, total);
+    else bwd::dkdv_kernel<<<dim3((unsigned)total), bwd::kDkWaves * 64, 0, st>>>(p, nkblk);
     if (int rc = check_launch("attn_bwd dkdv")) return rc;
-    if (p.nsplit > 1) {
-      const int64_t threads = (int64_t)per_split * bwd::kDkParts * 16 * 32;
-      bwd::dkdv_combine_kernel<<<dim3((unsigned)(threads / 256)), 256, 0, st>>>(p, nkblk, per_split);
+    if (p.split_items > 0) {
+      const int64_t threads = (int64_t)p.split_items * bwd::kDkParts * 16 * 32;
+      bwd::dkdv_combine_kernel<<<dim3((unsigned)(threads / 256)), 256, 0, st>>>(p, nkblk);
       if (int rc = check_launch("attn_bwd dkdv combine")) return rc;
     }
   }

@@ -383,16 +383,14 @@ struct DkWave {
 };
 
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void dkdv1w_kernel(Params p, int nkblk, int total_blocks) {
+void dkdv1w_kernel(Params p, int nkblk) {
   __shared__ __attribute__((aligned(1024))) bf16 ring[kStages * 2 * kTileElems];
   __shared__ __attribute__((aligned(1024))) float stat[kStages * kStat];
 
-  const int logical = xcd_remap(blockIdx.x, total_blocks);
-  const int per_split = total_blocks / p.nsplit;
-  const int split = logical / per_split;
-  const int rest = logical - split * per_split;
-  const int kblk = rest % nkblk;
-  const int bh = rest / nkblk;
+  int item, split, rec;
+  dkdv_item(p, blockIdx.x, item, split, rec);
+  const int kblk = item % nkblk;
+  const int bh = item / nkblk;
   const int b = bh / p.H, h = bh - (bh / p.H) * p.H;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -400,7 +398,7 @@ void dkdv1w_kernel(Params p, int nkblk, int total_blocks) {
   const int key0 = kblk * kKeysPerWg + wave * 32;
 
   // Query tiles tq0 .. tq0 + ntiles - 1 (all of them without a split).
-  const int tper = (p.ntq + p.nsplit - 1) / p.nsplit;
+  const int tper = rec < 0 ? p.ntq : (p.ntq + p.nsplit - 1) / p.nsplit;
   const int tq0 = min(split * tper, p.ntq);
   const int ntiles = min(tper, p.ntq - tq0);
   const float* statb = p.stats + ((int64_t)bh * p.ntq + tq0) * kStat;
@@ -496,10 +494,10 @@ void dkdv1w_kernel(Params p, int nkblk, int total_blocks) {
   __syncthreads();  // every wave is done with the ring; no DMA in flight
 
   w.fence_acc();
-  if (p.nsplit > 1) {
+  if (rec >= 0) {
     // Partial accumulators: record wave (dV^T) and 4 + wave (dK^T), 16
     // coalesced 1 KB stores each.
-    f32x4* dst = reinterpret_cast<f32x4*>(p.part) + ((int64_t)logical * kDkParts + wave) * 16 * 64 + lane;
+    f32x4* dst = reinterpret_cast<f32x4*>(p.part) + ((int64_t)rec * kDkParts + wave) * 16 * 64 + lane;
     f32x4* dstk = dst + (int64_t)kWaves * 16 * 64;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -524,7 +522,7 @@ void dkdv1w_kernel(Params p, int nkblk, int total_blocks) {
 }  // namespace w1
 
 void launch_dkdv1w(const Params& p, int nkblk, int total, hipStream_t stream) {
-  w1::dkdv1w_kernel<<<dim3((unsigned)total), w1::kWaves * 64, 0, stream>>>(p, nkblk, total);
+  w1::dkdv1w_kernel<<<dim3((unsigned)total), w1::kWaves * 64, 0, stream>>>(p, nkblk);
 }
 
 }  // namespace bwd
