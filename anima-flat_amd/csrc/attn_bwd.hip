@@ -581,10 +581,11 @@ static bool stride_ok(const int64_t* s) {
 // fill at most half of the CUs, as the 128 items of the 512-key text context
 // at B = 2 and 16 heads or the last 32 of 2304 tokens' 288, each of them is
 // split over up to 4 workgroups of at least 4 query tiles. Behind whole
-// rounds the split has to save kDkTailTiles tiles, what the partials and the
-// combine pass cost (~14 us): 2304 tokens 188 -> 163 us for the backward, 2560
-// 210 -> 192.
-constexpr int kDkTailTiles = 8;
+// rounds the split has to save kDkTailTiles tiles, what the partials' way
+// through memory and the combine pass cost: the backward at 2304 tokens 188 ->
+// 165 us, 2560 209 -> 192, 3072 258 -> 248; saving 12 tiles (B=2 1536) it took
+// 144 us against 140.
+constexpr int kDkTailTiles = 16;
 struct DkSplit {
   int full_items, split_items, nsplit;
 };

@@ -611,15 +611,19 @@ static int fwd_scratch(void** out) {
 // Which head_dim-128 kernel runs.
 //   2, the key-split kernel of attn_fwd_ks.hip (64 queries per workgroup, the
 //      keys split over its waves), where it takes least: problems whose 256-
-//      query items fill a fraction of the chip. Time in us of one round of a
-//      form = kRoundUs + its tiles per wave x kKsTileUs or kTileUs, plus
-//      kMergeUs for the partials' way through memory and the combine launch;
-//      the constants are fits to graph-timed calls on MI355X (16 heads, to
-//      within 10%). Measured against the other two: B=1 256 tokens 10.8 ->
-//      8.8 us, 512 19.8 -> 10.8, 768 20.3 -> 12.7, 1024 22.8 -> 15.3, B=2
-//      1024 31.8 -> 27.6, 1024 x 512 keys 19.4 -> 10.9; where the rule turns
-//      it down: 1280 tokens 29.4 against 27.7, 256 x 4096 keys 30.3 against
-//      23.0, 1024 x 64 keys 8.6 against 6.5.
+//      query items fill a fraction of the chip. Estimated time in us: a round
+//      of workgroups takes a constant plus its tiles per wave (the other
+//      kernels' tiles are up to 40% faster on a part-filled chip, whose clock
+//      is higher), and split items kMergeUs more for the partials' way through
+//      memory and the combine launch. The constants are fits to graph-timed
+//      calls on MI355X (16 heads, to within 10%). Measured against the other
+//      two: B=1 256 tokens 10.8 -> 8.8 us, 512 19.8 -> 10.8, 1024 22.8 ->
+//      15.3, B=2 1024 31.7 -> 29.0, 1024 x 512 keys 19.8 -> 11.3; where the
+//      rule turns it down: 1280 tokens 27.4 against 29.4, 1536 31.2 against
+//      34.5, B=2 700 23.3 against 24.8, 256 x 4096 keys 23.0 against 30.3,
+//      1024 x 64 keys 6.5 against 8.6. With key lengths, which only the device
+//      knows, one round at most (lengths 58 and 322 of 512, B=2: 300 queries
+//      16.3 -> 12.2, but 1000 21.4 -> 23.0).
 //   else up to kPingPongMaxSk keys 0, the two-group kernel of attn_fwd_pp.hip,
 //      which hides more of a work item's fixed costs, and beyond 1, this
 //      file's one-wave-per-SIMD kernel. At B = 1-2, 4096 queries: the
@@ -628,7 +632,8 @@ static int fwd_scratch(void** out) {
 // AA_FWD_KERNEL=pp|1w|ks forces one (tests run them on every shape); -1 for
 // another value.
 constexpr int64_t kPingPongMaxSk = 2048;
-constexpr double kRoundUs = 4.0, kTileUs = 1.78, kKsTileUs = 2.1, kMergeUs = 8.0;
+constexpr double kRoundUs = 4.0, kTileUs = 1.78, kMergeUs = 8.0;
+constexpr double kKsRoundUs = 4.6, kKsTileUs = 2.1;
 static int fwd_kernel_choice(int64_t B, const FwdParams& p) {
   const char* e = std::getenv("AA_FWD_KERNEL");
   if (e && *e) {
@@ -640,12 +645,16 @@ static int fwd_kernel_choice(int64_t B, const FwdParams& p) {
   }
   const int64_t ncu = std::max(device_cu_count(), 1), tiles = (p.Sk + kBN - 1) / kBN;
   const int64_t ks_blocks = B * p.H * ((p.Sq + kKsQueries - 1) / kKsQueries);
-  const double ks = (double)((ks_blocks + ncu - 1) / ncu) *
-                    (kRoundUs + kKsTileUs * (double)((tiles + 3) / 4));
-  double other = (double)((p.full_blocks + ncu - 1) / ncu) * (kRoundUs + kTileUs * (double)tiles);
+  const int64_t ks_rounds = (ks_blocks + ncu - 1) / ncu;
+  const double ks = (double)ks_rounds * (kKsRoundUs + kKsTileUs * (double)((tiles + 3) / 4));
+  const auto rounds_us = [&](int64_t blocks, int64_t n) {
+    const double fill = std::min(1.0, (double)blocks / (double)ncu);
+    return (double)((blocks + ncu - 1) / ncu) * (kRoundUs + kTileUs * (0.6 + 0.4 * fill) * (double)n);
+  };
+  double other = rounds_us(p.full_blocks, tiles);
   if (p.split_items > 0)
-    other += kRoundUs + kTileUs * (double)((tiles + p.nsplit - 1) / p.nsplit) + kMergeUs;
-  if (ks < other) return 2;
+    other += rounds_us((int64_t)p.split_items * p.nsplit, (tiles + p.nsplit - 1) / p.nsplit) + kMergeUs;
+  if (ks < other && (!p.seqused || ks_rounds == 1)) return 2;
   return p.Sk <= kPingPongMaxSk ? 0 : 1;
 }
 

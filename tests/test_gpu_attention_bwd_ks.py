@@ -58,9 +58,9 @@ def test_key_split_dq(pkg, monkeypatch, B, Sq, Sk, H):
 @pytest.mark.parametrize(
     "Sq,Sk,H",
     [
-        # 260 key blocks: the last 4 of them split over query ranges. 1040 dQ
-        # items: the last 16 key-split.
-        (1000, 100, 260),
+        # 260 key blocks: the last 4 of them split over query ranges. 1560 dQ
+        # items: the last 24 key-split.
+        (1400, 100, 260),
         # 260 dQ items, 4 of them key-split; too few query tiles to split dK/dV.
         (70, 128, 260),
     ],
