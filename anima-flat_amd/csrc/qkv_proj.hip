@@ -15,8 +15,8 @@
 // Main loop: waves of 64 tokens x WN columns (2 x WN/32 accumulators), over K
 // in stages of 64: the stage's X and W rows move L2 -> LDS by DMA
 // (global_load_lds_dwordx4, no registers) into a ring of two stages, one
-// ahead (each wave's share issued over the first k-steps of the stage before),
-// one barrier per stage. Each DMA instruction moves 8 rows x 128 bytes,
+// ahead (each wave's share issued over the first k-steps of the stage before;
+// TileD: four stages, three ahead), one barrier per stage. Each DMA instruction moves 8 rows x 128 bytes,
 // whole cache lines: with 16 rows x 64 bytes (half lines) per instruction the
 // same loads stream at well under half the rate, which bounded this kernel.
 // A stage in LDS is blocks of 8 rows x 64 k (1 KiB, one DMA instruction);
@@ -52,7 +52,7 @@ constexpr int kPK = 64;       // K per stage
 constexpr int kPKMin = 32;    // K granularity: a last stage may hold 32
 constexpr int kPGroupM = 4;   // token tiles per work-order group
 
-template <int MT, int NS, int WN, int PS>
+template <int MT, int NS, int WN, int PS, int RING>
 struct ProjTile {
   static constexpr int kMT = MT;                       // tokens per workgroup
   static constexpr int kNS = NS;                       // sections per workgroup
@@ -65,15 +65,14 @@ struct ProjTile {
   static constexpr int kBlocks = (MT + kN) / 8;        // 8-row DMA blocks per stage
   static constexpr int kBPW = kBlocks / kWaves;        // ... per wave
   static constexpr int kCB = WN / 32;                  // 32-column blocks per wave
-  static constexpr int kRingElems = 2 * kStageElems;
-  // The next stage's DMA of a wave goes out in this many parts, one per
-  // k-step from the first: the load path takes one instruction per ~11
-  // cycles, so 8 waves issuing 8-10 each at once hold most of them back from
-  // their MFMAs for up to ~900 cycles. Two parts: QKV B=1 99.6 -> 95.5 us
-  // (tile B), xq 64.7 -> 62.2 us (tile A); four parts were slower, and so was
-  // splitting at all with four waves (tile C, whose two workgroups per CU
-  // already overlap one's loads with the other's MFMAs).
-  static constexpr int kDmaParts = kWaves == 8 ? 2 : 1;
+  static constexpr int kRing = RING;                   // stages in the LDS ring
+  static constexpr int kRingElems = RING * kStageElems;
+  // A stage's DMA of a wave goes out in this many parts, one per k-step from
+  // the first: the load path takes one instruction per ~11 cycles, so waves
+  // issuing 8-10 each at once hold most of them back from their MFMAs. Two
+  // parts: QKV B=1 99.6 -> 95.5 us (tile B), xq 64.7 -> 62.2 us (tile A), xkv
+  // 16.3 -> 15.4 us (tile C); four parts were slower.
+  static constexpr int kDmaParts = 2;
   // Sections staged per epilogue pass (the ring holds the staged bf16 tiles).
   static constexpr int kPassSecs = PS;
   static_assert(MT % 64 == 0 && kN % WN == 0 && WN % 32 == 0, "wave tiling");
@@ -85,9 +84,13 @@ struct ProjTile {
 // The last argument is the sections staged per epilogue pass. TileB stages
 // one at a time: with two, a wave whose columns straddle the passes keeps
 // 128 accumulators live through the first pass's normalisation and spills.
-using TileA = ProjTile<256, 2, 128, 2>;  // 128 KiB ring
-using TileB = ProjTile<256, 3, 192, 1>;  // 160 KiB ring
-using TileC = ProjTile<128, 1, 64, 1>;   // 64 KiB ring, two workgroups per CU
+// TileD is TileC with three stages in flight instead of one, for grids that
+// give a CU one workgroup: with no second one to fill in, the 16 MFMAs per
+// wave and stage do not cover a stage's load latency.
+using TileA = ProjTile<256, 2, 128, 2, 2>;  // 128 KiB ring
+using TileB = ProjTile<256, 3, 192, 1, 2>;  // 160 KiB ring
+using TileC = ProjTile<128, 1, 64, 1, 2>;   // 64 KiB ring, two workgroups per CU
+using TileD = ProjTile<128, 1, 64, 1, 4>;   // 128 KiB ring
 
 // The projection's output columns are nseg segments of H sections of 128:
 // segment g goes to out[g] ([ntok, H, 128]), RMS-normalised with weight nw[g]
@@ -144,34 +147,48 @@ __global__ __launch_bounds__(T::kThreads) void qkv_proj_kernel(ProjParams p) {
   const int dchunk0 = (lane & 7) ^ drow;  // even blocks
   const int dchunk1 = dchunk0 ^ 1;        // odd blocks
 
-  // Stage s -> ring slot s & 1: MT / 8 X blocks then kN / 8 W blocks,
+  // Stage s -> ring slot s % kRing: MT / 8 X blocks then kN / 8 W blocks,
   // contiguous (block b at b * 512); wave w moves blocks w G .. w G + G - 1.
-  // A last stage of 32 k (K % 64 == 32) loads chunks 4..7 from chunks 0..3
-  // (in bounds; those products are not computed).
-  // Blocks lo .. hi - 1 of the wave's share of stage s.
-  auto issue = [&](int s, int lo, int hi) {
-    bf16* st = lds + (s & 1) * T::kStageElems;
-    const int k0 = s * kPK;
-    const int cmask = p.K - k0 >= kPK ? 7 : 3;
+  // Per block the row base (scalar) and the lanes' byte offsets from it are
+  // computed once, so that a DMA instruction costs its base's advance along K
+  // and M0 only: with the addresses formed at each issue, from LDS pointers,
+  // the ~10 scalar instructions before each of a stage's 8-10 loads held up
+  // the wave's first MFMAs (xkv 17.3 -> 16.3 us, xq at 1024 tokens 22.9 ->
+  // 22.0, QKV at B=2 171.4 -> 169.6).
+  const bf16* sbase[T::kBPW];
+  uint32_t voff[T::kBPW];
 #pragma unroll
-    for (int i = 0; i < T::kBPW; ++i) {
-      if (i < lo || i >= hi) continue;
-      // Wave-uniform: block b, its first row b0 (clamped), the source matrix.
-      const int b = wave * T::kBPW + i;
-      const bool is_x = b < T::kMT / 8;
-      const int last = (is_x ? nrows : ncols) - 1;
-      const int b0 = min(8 * (is_x ? b : b - T::kMT / 8), last);
-      const int64_t rs = is_x ? p.xs : (int64_t)p.K;
-      const bf16* sbase = (is_x ? xbase : wbase) + b0 * rs + k0;
-      const uint32_t voff = (uint32_t)(min(drow, last - b0) * rs +
-                                       8 * (((i & 1) ? dchunk1 : dchunk0) & cmask)) * 2;
-      dma16_sv(sbase, voff, st + b * 512);
-    }
+  for (int i = 0; i < T::kBPW; ++i) {
+    // Wave-uniform: block b, its first row b0 (clamped), the source matrix.
+    const int b = wave * T::kBPW + i;
+    const bool is_x = b < T::kMT / 8;
+    const int last = (is_x ? nrows : ncols) - 1;
+    const int b0 = min(8 * (is_x ? b : b - T::kMT / 8), last);
+    const int64_t rs = is_x ? p.xs : (int64_t)p.K;
+    sbase[i] = (is_x ? xbase : wbase) + b0 * rs;
+    voff[i] = (uint32_t)(min(drow, last - b0) * rs + 8 * ((i & 1) ? dchunk1 : dchunk0)) * 2;
+  }
+  const uint32_t ring = lds_addr(lds) + (uint32_t)(wave * T::kBPW) * 1024u;
+  // A last stage of 32 k (K % 64 == 32) loads chunks 4..7 from chunks 0..3 (in
+  // bounds; those products are not computed): 64 bytes back.
+  const uint32_t back = (dchunk0 & 4) ? 64u : 0u;
+  // Blocks LO .. HI - 1 of the wave's share of stage s.
+  auto issue = [&](int s, auto lo, auto hi) {
+    constexpr int LO = decltype(lo)::value, HI = decltype(hi)::value;
+    const int k0 = s * kPK;
+    const uint32_t dst = ring + (uint32_t)((s % T::kRing) * T::kStageElems) * 2u;
+    const uint32_t adj = p.K - k0 >= kPK ? 0u : back;
+    static_for<LO, HI>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      dma16_sva_off<0, 1024 * i>(sbase[i] + k0, voff[i] - adj, dst);
+    });
   };
 
   const int nk = (p.K + kPK - 1) / kPK;
   const int nfull = p.K / kPK;  // stages of 64 k; a last one of 32 when K % 64 == 32
-  issue(0, 0, T::kBPW);
+  constexpr int kLead = T::kRing - 1;  // stages in flight
+  for (int s = 0; s < kLead && s < nk; ++s)
+    issue(s, std::integral_constant<int, 0>{}, std::integral_constant<int, T::kBPW>{});
 
   constexpr int kWavesM = T::kMT / 64;
   const int wm = wave % kWavesM;  // tokens 64 wm .. 64 wm + 63
@@ -201,12 +218,16 @@ __global__ __launch_bounds__(T::kThreads) void qkv_proj_kernel(ProjParams p) {
   constexpr int kPre = T::kCB <= 4 ? 2 : 1;
   auto stage = [&](int s, auto nsteps) {
     constexpr int NSTEPS = decltype(nsteps)::value;
-    // This wave's DMAs of stage s are done; the barrier publishes every
-    // wave's and retires all reads of stage s - 1, whose slot stage s + 1
+    // This wave's DMAs of stage s are done (the kLead - 1 stages after it may
+    // be in flight, while there are as many); the barrier publishes every
+    // wave's and retires all reads of stage s - 1, whose slot stage s + kLead
     // reuses.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (kLead > 1 && s + kLead - 1 < nk)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kLead - 1) * T::kBPW) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const bf16* stg = lds + (s & 1) * T::kStageElems;
+    const bf16* stg = lds + (s % T::kRing) * T::kStageElems;
     const bf16* xs = stg + wm * 4096;
     const bf16* ws = stg + T::kXElems + wn * (T::kWN / 8) * 512;
     bf16x8 a[NSTEPS][T::kCB], b[NSTEPS][2];
@@ -220,13 +241,16 @@ __global__ __launch_bounds__(T::kThreads) void qkv_proj_kernel(ProjParams p) {
 #pragma unroll
     for (int kk = 0; kk < kPre && kk < NSTEPS; ++kk) read(kk);
     constexpr int kParts = T::kDmaParts < NSTEPS ? T::kDmaParts : NSTEPS;
-    auto part = [&](int j) {
-      if (s + 1 < nk) issue(s + 1, j * T::kBPW / kParts, (j + 1) * T::kBPW / kParts);
+    auto part = [&](auto jj) {
+      constexpr int j = decltype(jj)::value;
+      if (s + kLead < nk)
+        issue(s + kLead, std::integral_constant<int, j * T::kBPW / kParts>{},
+              std::integral_constant<int, (j + 1) * T::kBPW / kParts>{});
     };
-    part(0);
-#pragma unroll
-    for (int kk = 0; kk < NSTEPS; ++kk) {
-      if (kk >= 1 && kk < kParts) part(kk);
+    part(std::integral_constant<int, 0>{});
+    static_for<0, NSTEPS>([&](auto KK) {
+      constexpr int kk = decltype(KK)::value;
+      if constexpr (kk >= 1 && kk < kParts) part(KK);
       if constexpr (kPre > 1) {
         if (kk + kPre < NSTEPS) read(kk + kPre);
       }
@@ -238,7 +262,7 @@ __global__ __launch_bounds__(T::kThreads) void qkv_proj_kernel(ProjParams p) {
         __builtin_amdgcn_sched_barrier(0);
         if (kk + 1 < NSTEPS) read(kk + 1);
       }
-    }
+    });
   };
   for (int s = 0; s < nfull; ++s) stage(s, std::integral_constant<int, kPK / 16>{});
   if (nk > nfull) stage(nfull, std::integral_constant<int, kPKMin / 16>{});
@@ -323,12 +347,15 @@ enum SegMode { kCopy = 0, kNorm = 1, kNormRope = 2 };
 // round. Round times measured on MI355X at K = 2048 (graph-timed): A 62-66 us,
 // B 87-97 us, C 40 us (two workgroups) -> weights 1.93, 2.85, 2 x 0.62. With
 // them the QKV projection at B = 2 takes two rounds of B (193.5 us) rather
-// than three of A (198.3 us, A/B on one box). Ties go to the lower index. The environment variable AA_PROJ_TILE = a, b or c
+// than three of A (198.3 us, A/B on one box). Ties go to the lower index. The environment variable AA_PROJ_TILE = a, b, c or d
 // forces a shape (all give identical results); any other value is an error
-// (-1).
-static int pick_tile(int64_t ntok, int64_t nsec) {
+// (-1). A TileC grid of at most one workgroup per CU takes TileD from K = 1536
+// on: at K = 2048 xq with 1024 tokens 21.2 -> 19.4 us, QKV with 512 26.2 ->
+// 21.0; at K = 1024 (xkv) the deeper fill costs what it gains, 15.5 against
+// 15.7.
+static int pick_tile(int64_t ntok, int64_t nsec, int64_t K) {
   if (const char* e = std::getenv("AA_PROJ_TILE")) {
-    if (e[0] && !e[1] && e[0] >= 'a' && e[0] <= 'c') return e[0] - 'a';
+    if (e[0] && !e[1] && e[0] >= 'a' && e[0] <= 'd') return e[0] - 'a';
     return -1;
   }
   const int64_t cus = std::max(1, device_cu_count());
@@ -350,6 +377,7 @@ static int pick_tile(int64_t ntok, int64_t nsec) {
       best_cost = cost;
     }
   }
+  if (best == 2 && K >= 1536 && (ntok + TileC::kMT - 1) / TileC::kMT * nsec <= cus) best = 3;
   return best;
 }
 
@@ -384,9 +412,9 @@ static int launch_proj(const char* what, const void* hid, int64_t hid_row_stride
   if (!aligned16(hid) || !aligned16(weight))
     return fail(AA_EINVAL, w + ": pointers must be 16-byte aligned");
   const int64_t ntok = B * S;
-  const int tile = pick_tile(ntok, nseg * H);
-  if (tile < 0) return fail(AA_EINVAL, "AA_PROJ_TILE must be a, b or c");
-  const int64_t mt = tile == 2 ? TileC::kMT : TileA::kMT;
+  const int tile = pick_tile(ntok, nseg * H, K);
+  if (tile < 0) return fail(AA_EINVAL, "AA_PROJ_TILE must be a, b, c or d");
+  const int64_t mt = tile >= 2 ? TileC::kMT : TileA::kMT;
   const int ns = tile == 0 ? TileA::kNS : tile == 1 ? TileB::kNS : TileC::kNS;
   const int64_t mtiles = (ntok + mt - 1) / mt;
   const int64_t total = mtiles * ((nseg * H + ns - 1) / ns);
@@ -411,7 +439,8 @@ static int launch_proj(const char* what, const void* hid, int64_t hid_row_stride
   p.eps = eps;
   if (tile == 0) qkv_proj_kernel<TileA><<<dim3((unsigned)total), TileA::kThreads, 0, st>>>(p);
   else if (tile == 1) qkv_proj_kernel<TileB><<<dim3((unsigned)total), TileB::kThreads, 0, st>>>(p);
-  else qkv_proj_kernel<TileC><<<dim3((unsigned)total), TileC::kThreads, 0, st>>>(p);
+  else if (tile == 2) qkv_proj_kernel<TileC><<<dim3((unsigned)total), TileC::kThreads, 0, st>>>(p);
+  else qkv_proj_kernel<TileD><<<dim3((unsigned)total), TileD::kThreads, 0, st>>>(p);
   return check_launch(what);
 }
 
