@@ -121,8 +121,8 @@ void dkdv_kernel(Params p, int nkblk) {
   dodma.setup(g, lane, p.s_do[1]);
   auto issue_tile = [&](int t) {
     const int st = t % kDkStages, q0 = (tq0 + t) * kT, nr = min(kT, p.Sq - q0);
-    qdma.issue(qbase + (int64_t)q0 * p.s_q[1], p.s_q[1], nr, rows[st][0], lane);
-    dodma.issue(dobase + (int64_t)q0 * p.s_do[1], p.s_do[1], nr, rows[st][1], lane);
+    qdma.issue(qbase + (int64_t)q0 * p.s_q[1], p.s_q[1], nr, lds_addr(rows) + (uint32_t)st * 32768u, lane);
+    dodma.issue(dobase + (int64_t)q0 * p.s_do[1], p.s_do[1], nr, lds_addr(rows) + (uint32_t)st * 32768u + 16384u, lane);
     if (wave == 4) dma16(statb + (int64_t)t * kStat + 4 * lane, stat[st]);
   };
 
@@ -427,14 +427,15 @@ void dq_kernel(Params p, int nqblk, int total_blocks) {
   // at each issue: held in registers they would push this kernel past 256.
   const int g = wave & 3;
   auto issue_tile = [&](int t) {
-    const int st = t % kDqStages, k0 = t * kT, nr = min(kT, p.Sk - k0);
+    const int k0 = t * kT, nr = min(kT, p.Sk - k0);
+    const uint32_t dst = lds_addr(tiles) + (uint32_t)(t % kDqStages) * 32768u;  // K tile, V tile
     // An opaque copy of the lane index keeps the compiler from hoisting the
     // offsets out of the tile loop (where they would hold registers again).
     int ln = lane;
     asm volatile("" : "+v"(ln));
-    DualDma::issue_quad(g, kbase + (int64_t)k0 * p.s_k[1], p.s_k[1], nr, tiles[st][0], ln,
+    DualDma::issue_quad(g, kbase + (int64_t)k0 * p.s_k[1], p.s_k[1], nr, dst, ln,
                         DualDma::lane_off(g, ln, p.s_k[1], 0), DualDma::lane_off(g, ln, p.s_k[1], 1));
-    DualDma::issue_quad(g, vbase + (int64_t)k0 * p.s_v[1], p.s_v[1], nr, tiles[st][1], ln,
+    DualDma::issue_quad(g, vbase + (int64_t)k0 * p.s_v[1], p.s_v[1], nr, dst + 16384u, ln,
                         DualDma::lane_off(g, ln, p.s_v[1], 0), DualDma::lane_off(g, ln, p.s_v[1], 1));
   };
 

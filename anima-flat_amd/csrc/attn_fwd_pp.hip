@@ -108,32 +108,36 @@ struct KVDma {
     voff = (uint32_t)(r * p.vs1 + vcol) * 2u;
   }
 
-  // Tile t (keys 64 t ..) of the (batch, head) at kp / vp into kd / vd.
+  // Tile t (keys 64 t ..) of the (batch, head) at kp / vp into the ring stage
+  // at LDS byte address `stage` (K tile, then V tile).
   __device__ __forceinline__ void issue(const FwdParams& p, const bf16* kp, const bf16* vp, int klen,
-                                        int t, bf16* kd, bf16* vd) const {
+                                        int t, uint32_t stage) const {
     const int kb = t * kBN;
     static_assert(kDmaPerWave == 4, "four DMA blocks per wave per tile");
+    const uint32_t kd = stage + 1024u * (uint32_t)b0, vd = kd + 16384u;
     if (kb + kBN <= klen) {
-#pragma unroll
-      for (int i = 0; i < kDmaPerWave; ++i) {
-        const int row0 = kb + rw + 8 * i;
-        dma16_sv(vp + (int64_t)row0 * p.vs1, voff, vd + (b0 + i) * 512);
-      }
-#pragma unroll
-      for (int i = 0; i < kDmaPerWave; ++i) {
-        const int row0 = kb + rw + 8 * i;
-        dma16_sv(kp + (int64_t)row0 * p.ks1, (i & 1) ? koff1 : koff0, kd + (b0 + i) * 512);
-      }
+      const bf16* kt = kp + (int64_t)(kb + rw) * p.ks1;
+      const bf16* vt = vp + (int64_t)(kb + rw) * p.vs1;
+      static_for<0, 4>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        dma16_sva_off<0, 1024 * i>(vt, voff, vd);
+        vt += 8 * p.vs1;
+      });
+      static_for<0, 4>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        dma16_sva_off<0, 1024 * i>(kt, (i & 1) ? koff1 : koff0, kd);
+        kt += 8 * p.ks1;
+      });
     } else {
 #pragma unroll
       for (int i = 0; i < kDmaPerWave; ++i) {
         const int r = min(kb + rbase + 8 * i, klen - 1);
-        dma16(vp + (int64_t)r * p.vs1 + vcol, vd + (b0 + i) * 512);
+        dma16_a(vp + (int64_t)r * p.vs1 + vcol, vd + 1024u * i);
       }
 #pragma unroll
       for (int i = 0; i < kDmaPerWave; ++i) {
         const int r = min(kb + rbase + 8 * i, klen - 1);
-        dma16(kp + (int64_t)r * p.ks1 + ((i & 1) ? kcol1 : kcol0), kd + (b0 + i) * 512);
+        dma16_a(kp + (int64_t)r * p.ks1 + ((i & 1) ? kcol1 : kcol0), kd + 1024u * i);
       }
     }
   }
@@ -383,7 +387,7 @@ void attn_fwd_pp_kernel(FwdParams p) {
   const bf16* kp = p.k + it.b * p.ks0 + it.h * p.ks2;
   const bf16* vp = p.v + it.b * p.vs0 + it.h * p.vs2;
   auto issue_tile = [&](int t) {
-    dma.issue(p, kp, vp, it.klen, t0 + t, kv_lds[t % kStages][0], kv_lds[t % kStages][1]);
+    dma.issue(p, kp, vp, it.klen, t0 + t, lds_addr(kv_lds) + (uint32_t)(t % kStages) * 32768u);
   };
 
   static_assert(kAhead >= 1 && kAhead <= 4, "lookahead");

@@ -72,6 +72,14 @@ __device__ __forceinline__ void dma16(const void* src, const void* lds_base) {
                : "memory", "m0");
 }
 
+// The same to an LDS byte address (lds_addr): from a pointer, the generic
+// address is formed and tested for null at every issue.
+__device__ __forceinline__ void dma16_a(const void* src, uint32_t lds_byte) {
+  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_byte);
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0)
+               : "memory", "m0");
+}
+
 // The same with a compile-time byte offset on the global address
 // (global_load_lds_dwordx4's immediate offset, 0 <= kOff < 4096): DMAs from
 // one base at fixed strides share one address computation. The instruction
@@ -268,24 +276,29 @@ struct DualDma {
     off0 = lane_off(g, lane, rs, 0);
     off1 = lane_off(g, lane, rs, 1);
   }
-  __device__ __forceinline__ void issue(const bf16* base, int64_t rs, int nrows, bf16* tile,
+  // `tile`: LDS byte address of the tile.
+  __device__ __forceinline__ void issue(const bf16* base, int64_t rs, int nrows, uint32_t tile,
                                         int lane) const {
     issue_quad(g, base, rs, nrows, tile, lane, off0, off1);
   }
   // The DMA itself, with the offsets given (kernels short of registers pass
   // lane_off(...) computed at the call instead of holding them).
   __device__ __forceinline__ static void issue_quad(int g, const bf16* base, int64_t rs, int nrows,
-                                                    bf16* tile, int lane, uint32_t o0, uint32_t o1) {
+                                                    uint32_t tile, int lane, uint32_t o0, uint32_t o1) {
     const int rw = 32 * (g & 1);
+    const uint32_t dst = tile + 4096u * (uint32_t)g;
     if (nrows >= kTileRows) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        dma16_sv(base + (int64_t)(rw + 8 * i) * rs, (i & 1) ? o1 : o0, tile + (4 * g + i) * 512);
+      const bf16* row = base + rw * rs;
+      static_for<0, 4>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        dma16_sva_off<0, 1024 * i>(row, (i & 1) ? o1 : o0, dst);
+        row += 8 * rs;
+      });
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = min(rw + 8 * i + (lane >> 3), nrows - 1);
-        dma16(base + (int64_t)r * rs + col(g, lane, i & 1), tile + (4 * g + i) * 512);
+        dma16_a(base + (int64_t)r * rs + col(g, lane, i & 1), dst + 1024u * i);
       }
     }
   }
