@@ -59,8 +59,11 @@ constexpr int kBN = 32;                    // keys per tile
 constexpr int kWaves = 4;                  // one per SIMD
 constexpr int kQPerWg = kWaves * 32;       // 128 queries per work item
 constexpr int kStages = 3;
-constexpr int kSub = 4096;                 // 32 rows x 128 bf16 = 8 KB
-constexpr int kStageElems = 2 * kChunks * kSub;  // K0 K1 K2 V0 V1 V2 = 48 KB
+constexpr int kHalves = 6;                 // 64-wide head-dim halves of the line tiles
+constexpr int kHalfElems = 32 * 64;        // 32 rows x 64 bf16 = 4 KB
+constexpr int kStageElems = 2 * kHalves * kHalfElems;  // K then V of 32 keys = 48 KB
+constexpr uint32_t kStageBytes = 2 * kStageElems;
+constexpr uint32_t kVBytes = kStageBytes / 2;  // V's offset in a stage
 constexpr int kDmaPerTile = 12;            // DMA instructions per wave per K or V tile
 constexpr int kMaxSplit = 8;
 constexpr float kRescaleThreshold = 8.0f;  // log2 units
@@ -85,21 +88,6 @@ struct Params {
   float* part_lse;  // [items * nsplit][128]
 };
 
-// DMA blocks 4 g .. 4 g + 3 of a row tile (not swizzled) whose row 0 is at
-// `base`: rows 16 g + (lane & 15), chunk 4 i + lq (lq = lane >> 4) for block
-// 4 g + i, at element 2048 g + 512 i + 8 lane of the tile. Rows at or past
-// nrows (>= 1) re-read row nrows - 1, finite data whose scores are masked.
-__device__ __forceinline__ void dma_row_quad(const bf16* base, int64_t rs, int nrows,
-                                             const bf16* lds_tile, int g, int lane) {
-  const int row = min(16 * g + (lane & 15), nrows - 1);
-  const bf16* src = base + (int64_t)row * rs + 8 * (lane >> 4);
-  const bf16* dst = lds_tile + 4 * g * 512;
-  dma16_off<0>(src, dst);
-  dma16_off<64>(src, dst + 512);
-  dma16_off<128>(src, dst + 1024);
-  dma16_off<192>(src, dst + 1536);
-}
-
 // Every MFMA is the compiler's builtin, so that the compiler pads the hazards
 // between an MFMA and the VALU code around it (a VALU write to an MFMA's
 // source registers right after its issue corrupts its operands; the
@@ -110,18 +98,20 @@ __device__ __forceinline__ void mfma_o(f32x16& acc, bf16x8 a, bf16x8 b) {
   acc = mfma32(a, b, acc);
 }
 
-// One tile's DMA work of one wave: three quads of 4 DMA instructions (16
-// rows x 4 chunks of 8 columns each), issued one instruction per MFMA slot of
-// phase 1. A wave with no tile left to move issues the same 12 instructions
-// into a dummy LDS area instead, so that every wave issues exactly 12 per
-// tile and one vmcnt(12) is the wait everywhere.
+// One tile's DMA work of one wave: 12 blocks of 8 rows x 64 columns (whole
+// cache lines), row groups rg = 0..3 of three 64-wide halves, one instruction
+// every four MFMA slots. The halves of a row group share its address. A wave
+// with no tile left to move issues the same 12 instructions into a dummy LDS
+// area instead, so that every wave issues exactly 12 per tile and one
+// vmcnt(12) is the wait everywhere.
 struct DmaJob {
-  const bf16* src[3];  // this lane's global address of quad q (offsets 64 i bytes follow)
-  const bf16* dst[3];  // LDS destination of quad q (blocks at + 512 i elements)
+  const bf16* src[4];  // this lane's address of row group rg (half j at + 128 j bytes)
+  uint32_t dst;        // LDS byte address (block (j, rg) at + 1024 (4 j + rg))
 
   template <int i>
   __device__ __forceinline__ void issue() const {
-    dma16_off<64 * (i & 3)>(src[i >> 2], dst[i >> 2] + 512 * (i & 3));
+    constexpr int j = i >> 2, rg = i & 3;
+    dma16_off<128 * j, 1024 * i>(src[rg], dst);
   }
 };
 
@@ -150,14 +140,15 @@ struct Wave {
   f32x4 lsum;       // row sum of query li (all four elements), by MFMA
   bf16x8 sel;       // 0/1 selector: the A operand of the row-sum MFMA
   float c, thr_raw;
-  int li, hh, k_rd, v_tr0, v_tr1;
+  int li, hh, k_rd[4], v_tr0, v_tr1;
 
   __device__ __forceinline__ void setup(int lane, float c_) {
     li = lane & 31;
     hh = lane >> 5;
-    k_rd = row_rd(lane);
-    v_tr0 = swz_tr_rd(lane, 0);
-    v_tr1 = swz_tr_rd(lane, 1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) k_rd[j] = 2 * line_k_rd(lane, j);
+    v_tr0 = 2 * line_v_tr(lane, 0);
+    v_tr1 = 2 * line_v_tr(lane, 1);
     c = c_;
     thr_raw = kRescaleThreshold / c;
     // Zeros pinned into AGPRs, the file every later MFMA keeps O in.
@@ -180,42 +171,47 @@ struct Wave {
     for (int i = 0; i < 8; ++i) sel[i] = one;
   }
 
-  // Operand reads address LDS as one pinned 32-bit byte base per tile (two
-  // for the transposed V^T reads) plus compile-time offsets, which fold into
-  // the instructions' immediate field; computed per operand, the addresses
-  // would take a VGPR each and push the Q^T operands out to scratch.
+  // Operand reads address LDS as pinned 32-bit byte bases per tile (four for
+  // the K reads, one per chunk pair of a half; two for the transposed V^T
+  // reads, one per parity of the 32-column block) plus compile-time offsets,
+  // which fold into the instructions' immediate field; computed per operand,
+  // the addresses would take a VGPR each and push the Q^T operands out to
+  // scratch.
   //
-  // K operand kk (head-dim 16 kk .. 16 kk + 15) of the tile whose K starts at
-  // byte address kb: sub-tile kk / 8, chunk pair kk % 8.
+  // K operand kk (head-dim 16 kk .. 16 kk + 15): half kk / 4, chunk pair kk % 4.
   template <int kk>
-  __device__ __forceinline__ bf16x8 k_op(uint32_t kb) const {
-    return lds_ld16(kb + 2 * ((kk >> 3) * kSub + 256 * (kk & 7)));
+  __device__ __forceinline__ bf16x8 k_op(const uint32_t (&kb)[4]) const {
+    return lds_ld16(kb[kk & 3] + 2 * kHalfElems * (kk >> 2));
   }
-  __device__ __forceinline__ uint32_t k_base(const bf16* kst) const {
-    uint32_t b = lds_addr(kst + k_rd);
-    asm volatile("" : "+v"(b));
-    return b;
+  __device__ __forceinline__ void k_bases(uint32_t kst, uint32_t (&kb)[4]) const {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      kb[j] = kst + (uint32_t)k_rd[j];
+      asm volatile("" : "+v"(kb[j]));
+    }
   }
-  // V^T operand of PV op i (d-block db = i % 12, key chunk c4 = i / 12) of the
-  // tile whose V starts at vst: bases vb0 / vb1 of the two transposed reads.
+  // V^T operand of PV op i (d-block db = i % 12, key chunk c4 = i / 12): the
+  // two transposed reads are one row group (1 KB) apart.
   template <int i>
   __device__ __forceinline__ bf16x8 v_op(uint32_t vb0, uint32_t vb1) const {
     constexpr int db = i % 12, c4 = i / 12;
-    constexpr uint32_t off = 2 * ((db >> 2) * kSub + 2048 * c4 + 512 * (db & 3));
-    const s16x4 lo = lds_ld8_tr(vb0 + off);
-    const s16x4 hi = lds_ld8_tr(vb1 + off);
+    constexpr uint32_t off = 2 * (kHalfElems * (db >> 1) + 1024 * c4);
+    const uint32_t vb = (db & 1) ? vb1 : vb0;
+    const s16x4 lo = lds_ld8_tr(vb + off);
+    const s16x4 hi = lds_ld8_tr(vb + off + 1024);
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   }
-  __device__ __forceinline__ void v_bases(const bf16* vst, uint32_t& vb0, uint32_t& vb1) const {
-    vb0 = lds_addr(vst + v_tr0);
-    vb1 = lds_addr(vst + v_tr1);
+  __device__ __forceinline__ void v_bases(uint32_t vst, uint32_t& vb0, uint32_t& vb1) const {
+    vb0 = vst + (uint32_t)v_tr0;
+    vb1 = vst + (uint32_t)v_tr1;
     asm volatile("" : "+v"(vb0), "+v"(vb1));
   }
 
   // S^T of a tile without interleaved work (the first tile of a range).
-  __device__ __forceinline__ void qk_plain(const bf16* kst, f32x16& acc) {
+  __device__ __forceinline__ void qk_plain(uint32_t kst, f32x16& acc) {
     bf16x8 q[kPf];
-    const uint32_t kb = k_base(kst);
+    uint32_t kb[4];
+    k_bases(kst, kb);
     static_for<0, 24 + kPf>([&](auto I) {
       constexpr int i = decltype(I)::value;
       if constexpr (i >= kPf) {
@@ -257,11 +253,12 @@ struct Wave {
   // Phase 1: S^T of the next tile (kst, skipped when QK is false) with P of
   // the current tile s -> pb and the row sums in the same slots.
   template <bool QK>
-  __device__ __forceinline__ void phase1(const bf16* kst, const DmaJob& job) {
+  __device__ __forceinline__ void phase1(uint32_t kst, const DmaJob& job) {
     const float mc = m_raw * c;
     bf16x8 q[kPf];
     float pf = 0.f;
-    const uint32_t kb = QK ? k_base(kst) : 0u;
+    uint32_t kb[4];
+    if constexpr (QK) k_bases(kst, kb);
     static_for<0, 24 + kPf>([&](auto I) {
       constexpr int i = decltype(I)::value;
       if constexpr (QK && i >= kPf) {
@@ -295,7 +292,7 @@ struct Wave {
   // Phase 2: O^T += V^T P^T of the current tile (vst) with the row max of the
   // next tile sn (when MAX) in the first slots.
   template <bool MAX>
-  __device__ __forceinline__ void phase2(const bf16* vst, const DmaJob& job) {
+  __device__ __forceinline__ void phase2(uint32_t vst, const DmaJob& job) {
     bf16x8 q[kPf];
     float ma = 0.f, mb = 0.f;
     uint32_t vb0, vb1;
@@ -357,9 +354,9 @@ struct Wave {
 // and share its K/V tiles in that XCD's L2.
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void attn_fwd_d384_kernel(Params p) {
-  // The ring, then 4 KB that DMAs with nothing to move write into.
-  __shared__ __attribute__((aligned(1024))) bf16 lds[kStages * kStageElems + 2048];
-  const bf16* dummy = lds + kStages * kStageElems;
+  // The ring, then 12 KB that DMAs with nothing to move write into.
+  __shared__ __attribute__((aligned(1024))) bf16 lds[kStages * kStageElems + 512 * kDmaPerTile];
+  const uint32_t ring = lds_addr(lds);
 
   const int L = xcd_remap(blockIdx.x, gridDim.x);
   const int split = L / p.items;
@@ -380,32 +377,34 @@ void attn_fwd_d384_kernel(Params p) {
 
   const bf16* kp = p.k + it.b * p.ks0 + it.h * p.ks2;
   const bf16* vp = p.v + it.b * p.vs0 + it.h * p.vs2;
-  auto stage = [&](int t) -> bf16* { return lds + (t % kStages) * kStageElems; };
+  auto stage = [&](int t) -> uint32_t { return ring + (uint32_t)(t % kStages) * kStageBytes; };
   const bool k_mover = wave < 2;
-  // DMA job of tile t: K (waves 0-1, row tile) or V (waves 2-3, swizzled row
-  // tile), 3 quads per wave: quad x = 0..5 of the tensor covers chunk x / 2,
-  // row group x % 2. Rows past the tile's keys re-read its last key (their
-  // scores are masked). t >= n gives the dummy job.
+  // DMA job of tile t: halves 3 mw .. 3 mw + 2 of K (waves 0-1) or V (waves
+  // 2-3). Rows past the tile's keys re-read its last key (their scores are
+  // masked). t >= n gives the dummy job.
+  const int mw = k_mover ? wave : wave - 2;
+  const bf16* mbase = (k_mover ? kp : vp) + 192 * mw;
+  const int64_t mrs = k_mover ? p.ks1 : p.vs1;
+  const int mchunk[2] = {8 * (k_mover ? line_k_chunk(lane, 0) : line_v_chunk(lane)),
+                         8 * (k_mover ? line_k_chunk(lane, 1) : line_v_chunk(lane))};
+  int64_t moff[4];  // of a whole tile's row groups
+#pragma unroll
+  for (int rg = 0; rg < 4; ++rg) moff[rg] = (8 * rg + (lane >> 3)) * mrs + mchunk[rg & 1];
   auto job_of = [&](int t) -> DmaJob {
     DmaJob j;
-    const int lq = lane >> 4;
+    const bool live = t < n;
+    const int kb = live ? (t0 + t) * kBN : 0;
+    const int nrows = live ? it.klen - kb : 1;
+    const bf16* base = mbase + (int64_t)kb * mrs;
+    j.dst = live ? stage(t) + (k_mover ? 0u : kVBytes) + kDmaPerTile * 1024u * (uint32_t)mw
+                 : ring + kStages * kStageBytes;
+    if (nrows >= kBN) {
 #pragma unroll
-    for (int qd = 0; qd < 3; ++qd) {
-      if (t >= n) {
-        j.src[qd] = kp + 8 * lq;
-        j.dst[qd] = dummy;
-        continue;
-      }
-      const int kb = (t0 + t) * kBN;
-      const int nrows = it.klen - kb;
-      const int x = 3 * (k_mover ? wave : wave - 2) + qd;
-      const int g = x & 1;
-      const int r = k_mover ? (lane & 15) : ((lane & 15) ^ (4 * lq));
-      const int row = min(16 * g + r, nrows - 1);
-      const bf16* base = k_mover ? kp + (int64_t)kb * p.ks1 : vp + (int64_t)kb * p.vs1;
-      const int64_t rs = k_mover ? p.ks1 : p.vs1;
-      j.src[qd] = base + (int64_t)row * rs + 128 * (x >> 1) + 8 * lq;
-      j.dst[qd] = stage(t) + ((k_mover ? 0 : kChunks) + (x >> 1)) * kSub + 4 * g * 512;
+      for (int rg = 0; rg < 4; ++rg) j.src[rg] = base + moff[rg];
+    } else {
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg)
+        j.src[rg] = base + (int64_t)min(8 * rg + (lane >> 3), nrows - 1) * mrs + mchunk[rg & 1];
     }
     return j;
   };
@@ -460,7 +459,7 @@ void attn_fwd_d384_kernel(Params p) {
       const bool more = t + 1 < n;
       const int kbn = (t0 + t + 1) * kBN;
       if (more && kbn + kBN > it.klen) w.mask(w.sn, kbn, it.klen);
-      w.phase2<true>(stage(t) + kChunks * kSub, job);
+      w.phase2<true>(stage(t) + kVBytes, job);
       if (more) w.update_max();
       w.s = w.sn;
     }

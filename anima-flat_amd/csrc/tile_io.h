@@ -3,20 +3,7 @@
 // Every streamed operand is a tile of 64 rows x 128 bf16 (16 KB): 64 keys or
 // queries, each with its 128 head-dim values. LDS has 64 banks of 4 bytes;
 // every format below keeps its operand reads free of bank conflicts. The
-// row tiles serve the head_dim-384 forward (32-row sub-tiles); the line tiles
-// further down serve the head_dim-128 forward and the backward.
-//
-// Row tile: element (r, d) at (r >> 4) * 2048 + (d >> 3) * 128 + (r & 15) * 8 + (d & 7),
-//   i.e. 256-byte slices of (16-row group, 16-byte chunk). An A-operand read
-//   of row 32 t + li, chunk 2 kk + hh (lane li = lane % 32, hh = lane / 32) is
-//   at row_rd(lane) + 4096 t + 256 kk: 16 lanes cover 16 consecutive slots.
-//
-// Swizzled row tile: the same with the row slot inside each slice XORed with
-//   4 * (chunk % 4): element (r, d) at
-//   (r >> 4) * 2048 + (d >> 3) * 128 + (((r & 15) ^ (4 * ((d >> 3) & 3))) * 8) + (d & 7).
-//   It can be read transposed with ds_read_b64_tr_b16 (swz_tr_rd): the 32
-//   lanes of one read touch 4 rows x 4 chunks, which land in 16 distinct
-//   slots.
+// head_dim-384 forward uses the line tiles with 32 rows per 64-wide half.
 //
 // Transposed operand: the A operand of v_mfma_f32_32x32x16_bf16 with the
 //   tile's rows as the k index, A[m][k] = tile(row k, column 32 dt + m) for
@@ -37,25 +24,6 @@ namespace aa {
 
 constexpr int kTileRows = 64;
 constexpr int kTileElems = kTileRows * 128;  // 16 KB of bf16
-
-// Per-lane read offset (elements) of a row-operand read of a row tile.
-__device__ __forceinline__ int row_rd(int lane) {
-  const int li = lane & 31, hh = lane >> 5;
-  return (li >> 4) * 2048 + (li & 15) * 8 + hh * 128;
-}
-
-// Per-lane offsets of the two ds_read_b64_tr_b16 reads (r2 = 0, 1) of a
-// transposed operand of a swizzled row tile. In a group of 16 lanes
-// (G = lane / 16), lanes 4 j .. 4 j + 3 (c = lane % 4) address the four
-// 8-byte pieces of row 16 c4 + 4 (G >> 1) + j + 8 r2, columns
-// 32 dt + 16 (G & 1) + 4 c .. + 3, and lane 16 G + i receives column
-// 32 dt + 16 (G & 1) + i of those four rows: A[m][k] with m = lane % 32 and
-// k = 8 (G >> 1) + 4 r2 + j, the accumulator row order.
-__device__ __forceinline__ int swz_tr_rd(int lane, int r2) {
-  const int G = lane >> 4, j = (lane >> 2) & 3, c = lane & 3;
-  const int slot = (((4 * (G >> 1) + j) ^ (4 * (c >> 1))) & 7) + 8 * (r2 ^ (G & 1));
-  return 256 * (G & 1) + 128 * (c >> 1) + 4 * (c & 1) + 8 * slot;
-}
 
 // Workgroup-wide DMA helpers ------------------------------------------------
 
@@ -80,19 +48,18 @@ __device__ __forceinline__ void dma16_a(const void* src, uint32_t lds_byte) {
                : "memory", "m0");
 }
 
-// The same with a compile-time byte offset on the global address
-// (global_load_lds_dwordx4's immediate offset, 0 <= kOff < 4096): DMAs from
-// one base at fixed strides share one address computation. The instruction
-// adds its offset to the LDS address as well (M0 + offset + 16 * lane), so M0
-// is set kOff bytes below the destination.
-template <int kOff>
-__device__ __forceinline__ void dma16_off(const void* src, const void* lds_base) {
+// From src + kOff to LDS at lds_byte + kLds + 16 * lane, with both constants in
+// the instructions: DMAs from one base at fixed strides share one address
+// computation (global_load_lds_dwordx4's immediate offset, 0 <= kOff < 4096;
+// the instruction adds it to the LDS address as well, so M0 is set that much
+// lower).
+template <int kOff, int kLds>
+__device__ __forceinline__ void dma16_off(const void* src, uint32_t lds_byte) {
   static_assert(kOff >= 0 && kOff < 4096, "immediate offset range");
-  const uint32_t m0 =
-      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void*)lds_base) - (uint32_t)kOff;
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off offset:%2" ::"v"(src), "s"(m0),
-               "n"(kOff)
-               : "memory", "m0");
+  const uint32_t base = __builtin_amdgcn_readfirstlane(lds_byte);
+  asm volatile("s_add_i32 m0, %1, %3\n\tglobal_load_lds_dwordx4 %0, off offset:%2" ::"v"(src),
+               "s"(base), "n"(kOff), "n"(kLds - kOff)
+               : "memory", "m0", "scc");
 }
 
 __device__ __forceinline__ void wait_dma() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
@@ -194,10 +161,12 @@ __device__ __forceinline__ int line_k_rd(int lane, int j) {
   return ((li >> 3) * 512 + (li & 7) * 64 + (hh ^ fk) * 8) ^ (16 * j);
 }
 
-// Transposed-read offsets of a V line tile (the pieces swz_tr_rd describes:
-// in a group of 16 lanes G = lane / 16, lanes 4 j + c address piece c of row
-// 16 c4 + 4 (G >> 1) + j + 8 r2, columns 32 dt + 16 (G & 1) + 4 c .. + 3):
-// the piece is at line_v_tr(lane, dt & 1) + 4096 (dt >> 1) + 1024 c4 + 512 r2.
+// Transposed-read offsets of a V line tile (two ds_read_b64_tr_b16, r2 = 0, 1,
+// per operand: in a group of 16 lanes G = lane / 16, lanes 4 j + c, c < 4,
+// address the 8-byte piece c of row 16 c4 + 4 (G >> 1) + j + 8 r2, columns
+// 32 dt + 16 (G & 1) + 4 c .. + 3, and lane 16 G + i receives column
+// 32 dt + 16 (G & 1) + i of those four rows: the accumulator row order): the
+// piece is at line_v_tr(lane, dt & 1) + 4096 (dt >> 1) + 1024 c4 + 512 r2.
 __device__ __forceinline__ int line_v_tr(int lane, int dt_odd) {
   const int G = lane >> 4, j = (lane >> 2) & 3, c = lane & 3;
   const int ri = 4 * (G >> 1) + j;
@@ -235,7 +204,7 @@ __device__ __forceinline__ int dual_row_rd(int lane, int j) {
   return ((li >> 3) * 512 + (li & 7) * 64 + (hh ^ f) * 8) ^ (16 * j);
 }
 
-// Transposed-read offsets (the pieces swz_tr_rd describes, rows 16 c4 +
+// Transposed-read offsets (the pieces line_v_tr describes, rows 16 c4 +
 // 4 (G >> 1) + j + 8 r2, columns 32 dt + 16 (G & 1) + 4 c .. + 3): the piece
 // is at dual_tr_rd(lane, dt & 1, r2) + 4096 (dt >> 1) + 1024 c4 + 512 r2.
 __device__ __forceinline__ int dual_tr_rd(int lane, int dt_odd, int r2) {
