@@ -404,25 +404,6 @@ void attn_fwd_pp_kernel(FwdParams p) {
   w.read_q(qstage, lane);
   __syncthreads();
   if (!group_a) __syncthreads();
-  // The Q rows of the block that follows this one on its XCD (blocks start
-  // one per CU and round) into L2, one word of each 128-byte line, by the
-  // waves that have no DMA to wait for: otherwise a round's Q rows all come in
-  // at once, before any of its work. B=2, 4096 x 512 keys 41.9 -> 40.2 us,
-  // lengths 58 / 322 27.3 -> 25.8, B=4 82.7 -> 76.1. (The one-wave kernel,
-  // whose rounds are longer, and dq_kernel, with three times the rows, got
-  // slower by it: 9216 tokens 544 -> 546 us, the backward of that call 133 ->
-  // 138.)
-  uint32_t ahead[2] = {0u, 0u};
-  const int next = (int)blockIdx.x + p.round_blocks;
-  if (!group_a && next < p.full_blocks) {
-    int nitem, nrec;
-    block_item(p, next, nitem, nrec);
-    const Item ni = decode_item(p, nitem);
-    const int row = min(ni.qblk * kQPerWg + (wave & 3) * 64 + lane, p.Sq - 1);
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(p.q + ni.b * p.qs0 + ni.h * p.qs2 + (int64_t)row * p.qs1);
-    ahead[0] = q[0];
-    ahead[1] = q[32];
-  }
   if (ntiles > 0) {
     w.mblock<false, true>(kv_lds[0][1], kv_lds[0][0]);
     __syncthreads();
@@ -441,7 +422,6 @@ void attn_fwd_pp_kernel(FwdParams p) {
     w.mblock<true, false>(kv_lds[(ntiles - 1) % kStages][1], kv_lds[0][0]);
   }
   if (group_a) __syncthreads();
-  asm volatile("" ::"v"(ahead[0]), "v"(ahead[1]));  // the only use of those words
   // Output staging: the two stages after the last tile's are free (group B
   // may still be reading the last tile's V in its final M block; nothing else
   // is read or in flight).
