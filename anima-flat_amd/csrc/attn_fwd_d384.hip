@@ -30,17 +30,22 @@
 //   followed by the (rare) lazy rescale of O and l when tile t+1 raised a
 //   row max by more than 8 in log2 units (as in the d=128 kernel).
 //
-// K/V staging: a 3-stage LDS ring of 48 KB stages (K and V of 32 keys as
-//   three 32-row x 128 sub-tiles each: K in the row-tile format, V in the
-//   swizzled one, tile_io.h), filled by DMA (global_load_lds_dwordx4). K of
-//   tile t+3 and V of tile t+2 are issued during tile t, one DMA instruction
-//   every four slots of both phases, so each half has two tiles of lead time;
-//   waves 0-1 move K, waves 2-3 move V. A DMA instruction holds its wave
-//   while the CU's load path is busy: with all 12 of a tile issued in
-//   consecutive slots of phase 1 (the four waves at once), phase 1 took
-//   ~2460 cycles for its 24 MFMAs against ~1150 for phase 2's; spread over
-//   both phases, 434 -> 403 us at 16384 tokens (staggering the four waves'
-//   slots instead was slower, 505 us).
+// K/V staging: a 3-stage LDS ring of 48 KB stages (K and V of 32 keys as line
+//   tiles with 32 rows per 64-wide half, tile_io.h), filled by DMA
+//   (global_load_lds_dwordx4, 8 rows x 128 bytes each). K of tile t+3 and V of
+//   tile t+2 are issued during phase 2 of tile t, one DMA instruction every
+//   two slots; waves 0-1 move K, waves 2-3 move V.
+//   What bounds it: one CU draws 48 KB per tile, 7.7 TB/s over the chip at
+//   1.6 us per tile. In row tiles (16 rows x 64 bytes per instruction, half
+//   cache lines) that was the rate the load path streams, and the DMA had to
+//   be spread over both phases (411 us at 16384 tokens; 434 us with all of it
+//   in phase 1). Line tiles move it at twice that rate: 389 us with the same
+//   placement. Phase 1 carries the softmax's VALU work and phase 2 almost
+//   none, so the DMA goes there: 382 us (other offsets over both phases 385,
+//   12 consecutive slots 393), and operands read 4 instead of 6 slots ahead
+//   (8: 392): 372-376 us, 1.1 PFLOP/s (one process, same bits). What remains is
+//   the LDS: 128 queries read every K and V operand four times, 192 KB per
+//   tile and CU beside 1536 cycles of MFMA work.
 #include <algorithm>
 #include <cmath>
 #include <string>
@@ -67,7 +72,7 @@ constexpr uint32_t kVBytes = kStageBytes / 2;  // V's offset in a stage
 constexpr int kDmaPerTile = 12;            // DMA instructions per wave per K or V tile
 constexpr int kMaxSplit = 8;
 constexpr float kRescaleThreshold = 8.0f;  // log2 units
-constexpr int kPf = 6;                     // operands read ahead of their MFMA
+constexpr int kPf = 4;                     // operands read ahead of their MFMA
 constexpr int kQA = 16;                    // Q^T operands kept in AGPRs (the rest in VGPRs)
 
 struct Params {
@@ -100,7 +105,7 @@ __device__ __forceinline__ void mfma_o(f32x16& acc, bf16x8 a, bf16x8 b) {
 
 // One tile's DMA work of one wave: 12 blocks of 8 rows x 64 columns (whole
 // cache lines), row groups rg = 0..3 of three 64-wide halves, one instruction
-// every four MFMA slots. The halves of a row group share its address. A wave
+// every two slots of phase 2. The halves of a row group share its address. A wave
 // with no tile left to move issues the same 12 instructions into a dummy LDS
 // area instead, so that every wave issues exactly 12 per tile and one
 // vmcnt(12) is the wait everywhere.
@@ -253,7 +258,7 @@ struct Wave {
   // Phase 1: S^T of the next tile (kst, skipped when QK is false) with P of
   // the current tile s -> pb and the row sums in the same slots.
   template <bool QK>
-  __device__ __forceinline__ void phase1(uint32_t kst, const DmaJob& job) {
+  __device__ __forceinline__ void phase1(uint32_t kst) {
     const float mc = m_raw * c;
     bf16x8 q[kPf];
     float pf = 0.f;
@@ -266,7 +271,6 @@ struct Wave {
         sn = mfma32(q[op % kPf], qreg[op], op == 0 ? f32x16{} : sn);
       }
       if constexpr (QK && i < 24) q[i % kPf] = this->template k_op<i>(kb);
-      if constexpr (QK && i % 4 == 2 && i / 4 < kDmaPerTile / 2) job.template issue<i / 4>();
       // P: one score per slot for slots 0-15, packed and summed in pairs.
       if constexpr (i < 16) {
         const float e = fast_exp2(fmaf(s[i], c, -mc));
@@ -305,7 +309,7 @@ struct Wave {
         mfma_o(o[db], q[op % kPf], pb[c4]);
       }
       if constexpr (i < 24) q[i % kPf] = this->template v_op<i>(vb0, vb1);
-      if constexpr (i % 4 == 2 && i / 4 < kDmaPerTile / 2) job.template issue<kDmaPerTile / 2 + i / 4>();
+      if constexpr (i % 2 == 1 && i / 2 < kDmaPerTile) job.template issue<i / 2>();
       if constexpr (MAX) {
         if constexpr (i == kPf) {
           ma = max3f(sn[0], sn[1], sn[2]);
@@ -455,7 +459,7 @@ void attn_fwd_d384_kernel(Params p) {
       asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
       __syncthreads();
       const DmaJob job = job_of(k_mover ? t + 3 : t + 2);
-      w.phase1<true>(stage(t + 1), job);
+      w.phase1<true>(stage(t + 1));
       const bool more = t + 1 < n;
       const int kbn = (t0 + t + 1) * kBN;
       if (more && kbn + kBN > it.klen) w.mask(w.sn, kbn, it.klen);
