@@ -201,7 +201,15 @@ struct DqWave {
         if constexpr (ktr_slot(j) == g) tq[j % kTrQ] = this->template k_tr<j>();
       });
       if constexpr (g < 32) {
-        if constexpr (NEXT) this->template x_mfma<NB, g>(rq[(g >> 1) % kRowQ]);
+        if constexpr (NEXT) {
+          this->template x_mfma<NB, g>(rq[(g >> 1) % kRowQ]);
+          // Anchored in its slot: left alone, the compiler moves these MFMAs
+          // down to where mask and the next block read them, all in a row
+          // behind the VALU work that they are meant to cover (backward at
+          // 512 x 4096 keys 84 -> 76 us, 2048 tokens 117-119 -> 112-116).
+          f32x16& acc = g < 16 ? dp[NB][g & 1] : s[NB][g & 1];
+          asm volatile("" : "+v"(acc));
+        }
       } else {
         constexpr int op = g - 32, j = op >> 1;
         mfma_acc(dq[j & 3][op & 1], tq[j % kTrQ], zb[j >> 2][op & 1]);

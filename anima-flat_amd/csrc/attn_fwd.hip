@@ -100,6 +100,9 @@ constexpr uint32_t kStageBytes = 2u * kTileElems * sizeof(bf16);  // K tile, the
 // re-read row Sk - 1: finite data, and rows at or past the key length have
 // their scores masked to -inf (P = 0).
 struct KVDma {
+  // Here S^T stays in its slots by itself, and held there the loop is slower
+  // (2304 tokens 54.8 -> 56.2 us).
+  static constexpr bool kAnchorS = false;
   uint32_t ko[4], vo[4];      // per-lane offsets of blocks 0-3 (those of a tile inside Sk
                               // unless `clamped`)
   bool clamped;
@@ -617,11 +620,11 @@ static int fwd_scratch(void** out) {
 //      is higher), and split items kMergeUs more for the partials' way through
 //      memory and the combine launch. The constants are fits to graph-timed
 //      calls on MI355X (16 heads, to within 10%). Measured against the other
-//      two: B=1 256 tokens 10.8 -> 8.8 us, 512 19.8 -> 10.8, 1024 22.8 ->
-//      15.3, B=2 1024 31.7 -> 29.0, 1024 x 512 keys 19.8 -> 11.3; where the
-//      rule turns it down: 1280 tokens 27.4 against 29.4, 1536 31.2 against
-//      34.5, B=2 700 23.3 against 24.8, 256 x 4096 keys 23.0 against 30.3,
-//      1024 x 64 keys 6.5 against 8.6. With key lengths, which only the device
+//      two: B=1 256 tokens 10.6 -> 8.8 us, 512 20.0 -> 10.5, 1024 22.0 ->
+//      14.3, B=2 1024 31.0 -> 27.3, 1024 x 512 keys 19.5 -> 11.0; where the
+//      rule turns it down: 1280 tokens 27.2 against 29.1, 1536 30.6 against
+//      31.9, B=2 700 22.8 against 23.4, 256 x 4096 keys 23.0 against 31.1,
+//      1024 x 64 keys 6.4 against 8.4. With key lengths, which only the device
 //      knows, one round at most (lengths 58 and 322 of 512, B=2: 300 queries
 //      16.3 -> 12.2, but 1000 21.4 -> 23.0).
 //   else up to kPingPongMaxSk keys 0, the two-group kernel of attn_fwd_pp.hip,

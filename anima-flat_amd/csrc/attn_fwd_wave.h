@@ -256,6 +256,7 @@ struct FwdWave {
   // mask_next) and, with TRACK, its row max to mt. `dma` issues the K/V DMA
   // in the slots (after_slot) and waits for it where the kernel does that in
   // the slots too (before_slot, ahead of the slot's operand reads).
+  // Dma::kAnchorS holds the S^T MFMAs in their slots by empty asm statements.
   // FSUM: the fp32 probabilities' row sums too (for an exact LSE).
   template <int SB, bool NEXT, bool TRACK, bool FSUM, class Dma>
   __device__ __forceinline__ void tile(uint32_t dstage, bool mask_next, int kb_next, int klen,
@@ -288,6 +289,7 @@ struct FwdWave {
         if constexpr (NEXT) {
           constexpr int j = g >> 1, kb = j >> 3, kk = j & 7, qb = g & 1;
           s[NB][kb][qb] = mfma32(kq[j % kKQ], qreg[qb][kk], kk == 0 ? f32x16{} : s[NB][kb][qb]);
+          if constexpr (Dma::kAnchorS) asm volatile("" : "+v"(s[NB][kb][qb]));
         }
       } else {
         constexpr int op = g - 32, pp = op >> 1, c4 = pp >> 2, dt = pp & 3, qb = op & 1;
