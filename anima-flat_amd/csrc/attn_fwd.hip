@@ -629,12 +629,17 @@ static int fwd_scratch(void** out) {
 //      16.3 -> 12.2, but 1000 21.4 -> 23.0).
 //   else up to kPingPongMaxSk keys 0, the two-group kernel of attn_fwd_pp.hip,
 //      which hides more of a work item's fixed costs, and beyond 1, this
-//      file's one-wave-per-SIMD kernel. At B = 1-2, 4096 queries: the
+//      file's one-wave-per-SIMD kernel. At 4096 queries, B = 1-2, the
 //      two-group kernel is 5-8% faster at 512 and 1024 keys, the two tie at
-//      2048, the one-wave kernel is ~3% faster at 4096.
+//      2048 to 2560, the one-wave kernel is 2-3% faster at 4096. With fewer
+//      queries than a whole round the line lies higher: self-attention of
+//      2112 tokens 47.6 us (two-group) against 50.1, 2304 51.7 against 54.2,
+//      2560 57.9 against 59.8, B=2 2304 91.6 against 94.5, 2560 107.5 against
+//      109.0, but 3072 76.1 against 76.4 and B=2 148.9 against 147.2; 4096 x
+//      2560 keys, the worst call below the line, 78.4 against 77.8.
 // AA_FWD_KERNEL=pp|1w|ks forces one (tests run them on every shape); -1 for
 // another value.
-constexpr int64_t kPingPongMaxSk = 2048;
+constexpr int64_t kPingPongMaxSk = 2560;
 constexpr double kRoundUs = 4.0, kTileUs = 1.78, kMergeUs = 8.0;
 constexpr double kKsRoundUs = 4.6, kKsTileUs = 2.1;
 static int fwd_kernel_choice(int64_t B, const FwdParams& p) {

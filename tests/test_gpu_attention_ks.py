@@ -92,3 +92,17 @@ def test_key_split_growing_scores(pkg, monkeypatch):
     eo, el = ref.attention_lse(q, k, v, None)
     parity(out, eo, name="out")
     parity(lse, el, **LSE_TOL, name="lse")
+
+
+@pytest.mark.parametrize("S,kernel", [(2049, "pp"), (2560, "pp"), (2561, "1w")])
+def test_kernel_by_key_length(pkg, monkeypatch, S, kernel):
+    """The default rule's kernel on both sides of the two-group kernel's longest key range:
+    the bits of that kernel when forced, and the oracle's values on some rows."""
+    g = torch.Generator().manual_seed(S)
+    q, k, v = (ref.bf16_normal((1, S, 16, 128), g) for _ in range(3))
+    d = [t.to("cuda", BF) for t in (q, k, v)]
+    out = pkg.attention(*d).view(1, S, 16, 128)
+    monkeypatch.setenv("AA_FWD_KERNEL", kernel)
+    assert torch.equal(pkg.attention(*d).view(1, S, 16, 128), out)
+    rows = [0, S // 2, S - 1]
+    parity(out[:, rows], ref.attention_sdpa(q[:, rows], k, v), name="rows")
