@@ -22,6 +22,7 @@
 // about 56 slots (2000 cycles) to arrive, and a wait for "all but the 22
 // youngest" (24 at slot 0) ahead of each quarter's first read covers exactly
 // the loads up to it.
+#include <cfloat>
 #include <type_traits>
 
 #include "attn_fwd_ks.h"
@@ -205,8 +206,11 @@ void attn_fwd_ks_kernel(FwdParams p, int nqblk, int total_blocks) {
     });
     if (b0) w.max_plain<1>();
     else w.max_plain<0>();
-    w.m_raw[0] = w.mt[0];
-    w.m_raw[1] = w.mt[1];
+    // Finite also where every score of the wave's first tile is -inf (keys
+    // masked by an infinity): s - m would be NaN there, the other waves' keys
+    // and this one's later tiles would be lost to it.
+    w.m_raw[0] = fmaxf(w.mt[0], -FLT_MAX);
+    w.m_raw[1] = fmaxf(w.mt[1], -FLT_MAX);
 
     auto run = [&](auto sb, auto next, int i) {
       constexpr int SB = decltype(sb)::value;
@@ -265,14 +269,15 @@ void attn_fwd_ks_kernel(FwdParams p, int nqblk, int total_blocks) {
       l[v] = st_l[v * kKsQueries + 32 * qb + li];
       mx = fmaxf(mx, m[v]);
     }
-    const bool any = mx > -INFINITY;
     float sum = 0.f, fsum = 0.f;
 #pragma unroll
     for (int v = 0; v < kWaves; ++v) {
-      const float a = any ? fast_exp2((m[v] - mx) * p.c) : 0.f;
+      const float a = m[v] > -INFINITY ? fast_exp2((m[v] - mx) * p.c) : 0.f;  // 0: no keys
       sum += l[v] * a;
       if constexpr (LSE) fsum += st_f[v * kKsQueries + 32 * qb + li] * a;
     }
+    // No key, or none with a weight: O = 0, LSE = -inf (a NaN sum goes on).
+    const bool any = sum != 0.f;
     scale[qb] = any ? fast_exp2((w.m_raw[qb] - mx) * p.c) / sum : 0.f;
     if constexpr (LSE) {
       lse[qb] = any ? (mx * p.c + __log2f(fsum)) * kLn2 : -INFINITY;

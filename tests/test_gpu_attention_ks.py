@@ -106,3 +106,25 @@ def test_kernel_by_key_length(pkg, monkeypatch, S, kernel):
     assert torch.equal(pkg.attention(*d).view(1, S, 16, 128), out)
     rows = [0, S // 2, S - 1]
     parity(out[:, rows], ref.attention_sdpa(q[:, rows], k, v), name="rows")
+
+
+@pytest.mark.parametrize("first,last", [(0, 64), (64, 128), (192, 256), (0, 256), (320, 500), (448, 500), (0, 500)])
+def test_key_split_infinite_scores(pkg, monkeypatch, first, last):
+    """Keys first .. last - 1 at a score of -inf, in steps of the 64-key tiles dealt to the
+    waves: a wave's first tile, its last, every wave's first, all. They weigh nothing; with no
+    other key the output is 0 and the LSE -inf, as for an empty key range."""
+    q, k, v = _inputs(1, 70, 500, 2, 40)
+    q[..., 0], k[..., 0] = 1.0, 0.0  # column 0 of a key: added to each of its scores
+    k[:, first:last] = 0.0
+    k[:, first:last, :, 0] = float("-inf")
+    monkeypatch.setenv("AA_FWD_KERNEL", "ks")
+    d = [t.to("cuda", BF) for t in (q, k, v)]
+    out, lse = torch.ops.anima_flat.fa_fwd(*d)
+    assert torch.equal(torch.ops.anima_flat.fa_fwd_nolse(*d), out)
+    if last - first == 500:
+        assert not out.any() and torch.isneginf(lse).all()
+        return
+    keep = [j for j in range(500) if not first <= j < last]
+    eo, el = ref.attention_lse(q, k[:, keep], v[:, keep], None)
+    parity(out, eo, name="out")
+    parity(lse, el, **LSE_TOL, name="lse")
