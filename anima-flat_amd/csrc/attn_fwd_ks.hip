@@ -123,6 +123,37 @@ struct WaveDma {
   }
 };
 
+// The wave's row sum of query 32 qb + lane % 32 again, in plain arithmetic, for
+// rows whose sum on the matrix pipe took in another row's NaN or infinity
+// (FwdWave::setup; their O did not). From the staged Q rows and K in memory,
+// half of the keys per lane of a pair; only runs where a row holds no finite
+// numbers.
+__device__ __forceinline__ float row_sum_again(const FwdParams& p, const WaveDma& dma, const bf16* stage,
+                                               int qb, int lane, int wave, int n, int klen, float m) {
+  const bf16* q = stage + qb * 4096;
+  const float mc = m * p.c;
+  float sum = 0.f;
+#pragma unroll 1
+  for (int i = 0; i < n; ++i) {
+    const int lo = (wave + kWaves * i) * kBN, hi = min(lo + kBN, klen);
+#pragma unroll 1
+    for (int key = lo + (lane >> 5); key < hi; key += 2) {
+      const bf16* kr = dma.kp + (int64_t)key * dma.ks1;
+      float s = 0.f;
+#pragma unroll 1
+      for (int ch = 0; ch < kD / 8; ++ch) {
+        float x[8], y[8];
+        unpack8(ld16(q + stage_at(lane & 31, ch)), x);
+        unpack8(ld16(kr + 8 * ch), y);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s = fmaf(x[e], y[e], s);
+      }
+      sum += round_bf16(fast_exp2(fmaf(s, p.c, -mc)));
+    }
+  }
+  return pair_sum(sum);
+}
+
 // LSE: something reads the log-sum-exp (an output, or the padding correction),
 // so the fp32 probabilities are summed on the VALU beside the row sums of the
 // MFMAs (3.5% of a call: 1024 tokens 16.2 -> 16.8 us).
@@ -238,6 +269,15 @@ void attn_fwd_ks_kernel(FwdParams p, int nqblk, int total_blocks) {
   }
   wait_dma();
   w.fence_o();
+  float lsum[2] = {w.lsum[0][0], w.lsum[1][0]};
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb) {
+    const bool again = !(lsum[qb] <= FLT_MAX);
+    if (__builtin_amdgcn_ballot_w64(again)) {
+      const float sum = row_sum_again(p, dma, stage, qb, lane, wave, n, klen, w.m_raw[qb]);
+      lsum[qb] = again ? sum : lsum[qb];
+    }
+  }
 
   // Merge: every wave's (m, l) through the staging area, O^T times its weight
   // in fp32 through the ring. Wave d sums head-dims 32 d .. 32 d + 31 over the
@@ -254,7 +294,7 @@ void attn_fwd_ks_kernel(FwdParams p, int nqblk, int total_blocks) {
     if constexpr (LSE) lf = pair_sum(w.lf[qb][0] + w.lf[qb][1]);
     if (hh == 0) {
       st_m[wave * kKsQueries + 32 * qb + li] = w.m_raw[qb];
-      st_l[wave * kKsQueries + 32 * qb + li] = w.lsum[qb][0];
+      st_l[wave * kKsQueries + 32 * qb + li] = lsum[qb];
       if constexpr (LSE) st_f[wave * kKsQueries + 32 * qb + li] = lf;
     }
   }

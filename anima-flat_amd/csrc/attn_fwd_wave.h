@@ -88,7 +88,8 @@ struct FwdWave {
     // query n (+16 for odd l / 16) over one half of the chunk's keys. With
     // A[m][k] = 1 where bit 2 of m equals bit 3 of k, D[m][n] sums query n
     // for m % 8 < 4 and query n + 16 otherwise, which puts the row sum of
-    // query li = lane % 32 in all four D values of lane `lane`.
+    // query li = lane % 32 in all four D values of lane `lane`. Column n holds
+    // both queries' P, so a NaN in one makes the sum of the other NaN too.
     {
       const bf16 one = (bf16)(((lane & 15) >> 2 & 1) == ((lane >> 4) & 1) ? 1.0f : 0.0f);
 #pragma unroll

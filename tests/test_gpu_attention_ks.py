@@ -128,3 +128,23 @@ def test_key_split_infinite_scores(pkg, monkeypatch, first, last):
     eo, el = ref.attention_lse(q, k[:, keep], v[:, keep], None)
     parity(out, eo, name="out")
     parity(lse, el, **LSE_TOL, name="lse")
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_key_split_rows_stay_apart(pkg, monkeypatch, value):
+    """Query rows that hold no finite number give NaN, every other row what it gives without
+    them (32 queries share an MFMA's columns)."""
+    q, k, v = _inputs(1, 100, 300, 2, 50)
+    monkeypatch.setenv("AA_FWD_KERNEL", "ks")
+    d = [t.to("cuda", BF) for t in (q, k, v)]
+    want, want_lse = torch.ops.anima_flat.fa_fwd(*d)
+    rows = [3, 40, 62, 99]
+    d[0][:, rows] = value
+    others = [j for j in range(100) if j not in rows]
+    out, lse = torch.ops.anima_flat.fa_fwd(*d)
+    nolse = torch.ops.anima_flat.fa_fwd_nolse(*d)
+    assert torch.equal(nolse.isnan(), out.isnan()) and torch.equal(nolse[:, others], out[:, others])
+    # Their row sums are taken again from scores summed in another order: O within a bf16 step.
+    assert torch.allclose(out[:, others].float(), want[:, others].float(), rtol=2.0**-7, atol=0)
+    assert torch.equal(lse[..., others], want_lse[..., others])
+    assert out[:, rows].isnan().all() and lse[..., rows].isnan().all()
