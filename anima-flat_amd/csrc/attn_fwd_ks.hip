@@ -51,25 +51,32 @@ struct WaveDma {
   int64_t ks1, vs1;         // token strides
   uint32_t ko[8], vo[8];    // per-lane byte offsets of the tile's 8-row blocks
   uint32_t lds;             // LDS byte address of the wave's K tile
-  int lo;                   // first key that the next tile counts
   const bf16 *kt, *vt, *v3; // first rows of the K tile and V tile (chunks 0-2; 3) being fetched
 
   // Rows at or past klen are never fetched (V may hold anything there, and 0
-  // times a NaN is one): a range shorter than a tile re-reads its last row,
-  // longer ones have no tile that reaches past it (row_of in the kernel).
-  __device__ __forceinline__ void setup(const FwdParams& p, const bf16* k, const bf16* v, int klen,
-                                        int lane, uint32_t lds_) {
+  // times a NaN is one): the wave's last tile re-reads its last row past it
+  // (rows_k, rows_v from their first fetch on; what follows is that tile again).
+  __device__ __forceinline__ void setup(const FwdParams& p, const bf16* k, const bf16* v, int lane,
+                                        uint32_t lds_) {
     kp = k;
     vp = v;
     ks1 = p.ks1;
     vs1 = p.vs1;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = min(8 * i + (lane >> 3), klen - 1);
-      ko[i] = (uint32_t)(r * p.ks1 + 8 * line_k_chunk(lane, i & 1)) * 2u;
-      vo[i] = (uint32_t)(r * p.vs1 + 8 * line_v_chunk(lane)) * 2u;
-    }
+    rows_k(lane, kBN - 1);
+    rows_v<0, 8>(lane, kBN - 1);
     lds = lds_;
+  }
+  // Row offsets of a tile whose rows past `last` re-read it (V: blocks I .. E - 1).
+  __device__ __forceinline__ void rows_k(int lane, int last) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      ko[i] = (uint32_t)(min(8 * i + (lane >> 3), last) * ks1 + 8 * line_k_chunk(lane, i & 1)) * 2u;
+  }
+  template <int I, int E>
+  __device__ __forceinline__ void rows_v(int lane, int last) {
+#pragma unroll
+    for (int i = I; i < E; ++i)
+      vo[i] = (uint32_t)(min(8 * i + (lane >> 3), last) * vs1 + 8 * line_v_chunk(lane)) * 2u;
   }
 
   // Instruction i (0-3) of K quarter q / V chunk c: 8 rows x 64 d into the
@@ -85,13 +92,8 @@ struct WaveDma {
     dma16_sva_off<128 * dh, kVOff + (8 * dh + blk) * 1024>(c == 3 ? v3 : vt, vo[blk], lds);
   }
 
-  // The next tile's keys run from `lo` (it may be moved back over earlier
-  // ones).
   template <int B, class W>
-  __device__ __forceinline__ void mask(W& w, int kb, int klen) const {
-    w.template mask<B>(kb, klen);
-    w.template mask_below<B>(kb, lo);
-  }
+  __device__ __forceinline__ void mask(W& w, int kb, int klen) const { w.template mask<B>(kb, klen); }
   template <int g>
   __device__ __forceinline__ void first_slot() const {
     constexpr int q = (g >> 3) - 1, i = (g & 7) >> 1;
@@ -187,20 +189,30 @@ void attn_fwd_ks_kernel(FwdParams p, int nqblk, int total_blocks) {
     }
   }
 
-  // The wave's i-th tile is key tile wave + 4 i. A tile that would reach past
-  // klen is moved back to end there, and its keys below lo_of, which the tiles
-  // before it count, are masked.
+  // The wave's i-th tile is key tile wave + 4 i; `part` is the one that klen
+  // ends in (-1: none). A tile past the wave's last re-reads the last one into
+  // places that nothing reads again: every tile issues the same number of DMA
+  // instructions.
   const int n = (ntiles - wave + kWaves - 1) / kWaves;  // 0 if the wave has none
   auto lo_of = [&](int i) { return (wave + kWaves * i) * kBN; };
-  auto row_of = [&](int i) { return min(lo_of(i), max(klen - kBN, 0)); };
-  // A tile past the wave's last re-reads the last one into places that
-  // nothing reads again: every tile issues the same number of DMA instructions.
+  const int part = n > 0 && lo_of(n - 1) + kBN > klen ? n - 1 : -1;
+  const int last = klen - lo_of(n - 1) - 1;  // its last row
   WaveDma dma;
   const uint32_t mine = lds_addr(lds) + (uint32_t)wave * kWaveBytes;
-  dma.setup(p, p.k + b * p.ks0 + h * p.ks2, p.v + b * p.vs0 + h * p.vs2, klen, lane,
-            mine);
-  auto k_tile = [&](int i) { dma.kt = dma.kp + (int64_t)row_of(min(i, n - 1)) * dma.ks1; };
-  auto v_tile = [&](int i) { return dma.vp + (int64_t)row_of(min(i, n - 1)) * dma.vs1; };
+  dma.setup(p, p.k + b * p.ks0 + h * p.ks2, p.v + b * p.vs0 + h * p.vs2, lane, mine);
+  auto k_tile = [&](int i) {
+    dma.kt = dma.kp + (int64_t)lo_of(min(i, n - 1)) * dma.ks1;
+    if (i == part) dma.rows_k(lane, last);
+  };
+  // V chunks 0-2 of tile i; chunk 3.
+  auto v_tile = [&](int i) {
+    dma.vt = dma.vp + (int64_t)lo_of(min(i, n - 1)) * dma.vs1;
+    if (i == part) dma.rows_v<0, 6>(lane, last);
+  };
+  auto v3_tile = [&](int i) {
+    dma.v3 = dma.vp + (int64_t)lo_of(i) * dma.vs1;
+    if (i == part) dma.rows_v<6, 8>(lane, last);
+  };
   if (n > 0) {
     k_tile(0);
     static_for<0, 16>([&](auto I) {
@@ -219,18 +231,17 @@ void attn_fwd_ks_kernel(FwdParams p, int nqblk, int total_blocks) {
     // As if a tile -1 came before: the K quarters of tile 1, then V chunks
     // 0-2 of tile 0.
     k_tile(1);
-    dma.lo = lo_of(0);
     const int b0 = (n - 1) & 1;  // the last tile's S^T is in buffer 0
     const bool m0 = lo_of(0) + kBN > klen;
     if (b0) {
       w.qk_first<1>(dma);
-      if (m0) dma.template mask<1>(w, row_of(0), klen);
+      if (m0) dma.template mask<1>(w, lo_of(0), klen);
     } else {
       w.qk_first<0>(dma);
-      if (m0) dma.template mask<0>(w, row_of(0), klen);
+      if (m0) dma.template mask<0>(w, lo_of(0), klen);
     }
     static_for<0, 4>([&](auto I) { dma.template issue_k<3, decltype(I)::value>(); });
-    dma.vt = v_tile(0);
+    v_tile(0);
     static_for<0, 12>([&](auto I) {
       constexpr int i = decltype(I)::value;
       dma.template issue_v<(i >> 2), (i & 3)>();
@@ -247,11 +258,10 @@ void attn_fwd_ks_kernel(FwdParams p, int nqblk, int total_blocks) {
       constexpr int SB = decltype(sb)::value;
       constexpr bool NEXT = decltype(next)::value;
       k_tile(i + 2);
-      dma.v3 = v_tile(i);
-      dma.vt = v_tile(i + 1);
-      const int lo = lo_of(i + 1), row = row_of(i + 1);
-      dma.lo = lo;
-      w.tile<SB, NEXT, true, LSE>(0, lo + kBN > klen, row, klen, dma);
+      v3_tile(i);
+      v_tile(i + 1);
+      const int lo = lo_of(i + 1);
+      w.tile<SB, NEXT, true, LSE>(0, lo + kBN > klen, lo, klen, dma);
       if constexpr (NEXT) w.update_max<LSE>();
     };
     using I0 = std::integral_constant<int, 0>;

@@ -153,20 +153,6 @@ struct FwdWave {
           if (key >= klen) s[B][kt][qb][r] = -INFINITY;
         }
   }
-  // The same for keys below lo (a tile moved back over the keys before it).
-  template <int B>
-  __device__ __forceinline__ void mask_below(int kb, int lo) {
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kb + 32 * kt + 8 * (r >> 2) + 4 * hh + (r & 3);
-          if (key < lo) s[B][kt][qb][r] = -INFINITY;
-        }
-  }
-
   // Max step k (0..15) of S^T buffer B: block kb = k >> 3, query block
   // qb = k & 1, registers 4 ((k >> 1) & 3) .. + 3, into mx[qb].
   template <int B, int k>

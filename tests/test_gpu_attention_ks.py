@@ -1,7 +1,7 @@
 """GPU parity of the key-split forward (one workgroup per 64 queries, the keys
 split over its four waves and merged in LDS) against the CPU oracle, at the
-edges of its tiles: query blocks of 64, key tiles of 64 dealt to 4 waves, tiles
-moved back to end at the key length, waves without keys."""
+edges of its tiles: query blocks of 64, key tiles of 64 dealt to 4 waves, a last
+tile that re-reads its last row, waves without keys."""
 
 from __future__ import annotations
 
@@ -30,7 +30,7 @@ def _inputs(B, Sq, Sk, H, seed):
     [
         (1, 1, 1, 1, None),
         (1, 63, 64, 2, None),  # one key tile: three waves hold no keys
-        (2, 64, 65, 3, None),  # two tiles, the second moved back over 63 keys
+        (2, 64, 65, 3, None),  # two tiles, the second of one key
         (1, 65, 255, 2, None),  # every wave one tile, the last partial
         (1, 100, 256, 1, None),
         (1, 129, 257, 2, None),  # a second round of tiles for wave 0 only
@@ -148,3 +148,17 @@ def test_key_split_rows_stay_apart(pkg, monkeypatch, value):
     assert torch.allclose(out[:, others].float(), want[:, others].float(), rtol=2.0**-7, atol=0)
     assert torch.equal(lse[..., others], want_lse[..., others])
     assert out[:, rows].isnan().all() and lse[..., rows].isnan().all()
+
+
+@pytest.mark.parametrize("Sk,key", [(130, 120), (130, 3), (700, 638), (50, 20)])
+def test_key_split_infinite_value(pkg, monkeypatch, Sk, key):
+    """An infinite value makes its column infinite, not NaN, also near the end of a key range
+    that is no whole number of tiles."""
+    q, k, v = (t.to("cuda", BF) for t in _inputs(1, 70, Sk, 2, 60))
+    monkeypatch.setenv("AA_FWD_KERNEL", "ks")
+    want = torch.ops.anima_flat.fa_fwd_nolse(q, k, v)
+    v[:, key, :, 5] = float("inf")
+    out = torch.ops.anima_flat.fa_fwd_nolse(q, k, v)
+    assert torch.isposinf(out[..., 5]).all()
+    out[..., 5] = want[..., 5]
+    assert torch.equal(out, want)
