@@ -627,19 +627,23 @@ static int fwd_scratch(void** out) {
 //      1024 x 64 keys 6.4 against 8.4. With key lengths, which only the device
 //      knows, one round at most (lengths 58 and 322 of 512, B=2: 300 queries
 //      16.3 -> 12.2, but 1000 21.4 -> 23.0).
-//   else up to kPingPongMaxSk keys 0, the two-group kernel of attn_fwd_pp.hip,
-//      which hides more of a work item's fixed costs, and beyond 1, this
+//   else 0, the two-group kernel of attn_fwd_pp.hip, which hides more of a work
+//      item's fixed costs, up to kPingPongMaxSk keys, and beyond them 1, this
 //      file's one-wave-per-SIMD kernel. At 4096 queries, B = 1-2, the
 //      two-group kernel is 5-8% faster at 512 and 1024 keys, the two tie at
-//      2048 to 2560, the one-wave kernel is 2-3% faster at 4096. With fewer
-//      queries than a whole round the line lies higher: self-attention of
-//      2112 tokens 47.6 us (two-group) against 50.1, 2304 51.7 against 54.2,
-//      2560 57.9 against 59.8, B=2 2304 91.6 against 94.5, 2560 107.5 against
-//      109.0, but 3072 76.1 against 76.4 and B=2 148.9 against 147.2; 4096 x
-//      2560 keys, the worst call below the line, 78.4 against 77.8.
+//      2048 to 2560, the one-wave kernel is 2-3% faster at 4096. In a part-
+//      filled round the line lies at kPingPongPartMaxSk keys, for fewer than
+//      1.75 rounds of work items and no whole number of them: 144 items (2304
+//      tokens x 16 heads) 52.5 us (two-group) against 55.0, 160 (2560) 57.1
+//      against 59.7, 288 x 2304 keys 90.9 against 93.6, 432 x 2560 135.6
+//      against 137.1; but 256 x 2560 77.8 against 77.1, 504 x 2560 150.2 against
+//      148.4, and from two rounds on, where the one-wave kernel runs in its
+//      first-tile-max form, B=8 2304 tokens 314 against 307 and 2560 372
+//      against 361. At 3072 keys 144 items still gain 4%, 288 1% (113.6
+//      against 114.8), 432 lose 0.6%.
 // AA_FWD_KERNEL=pp|1w|ks forces one (tests run them on every shape); -1 for
 // another value.
-constexpr int64_t kPingPongMaxSk = 2560;
+constexpr int64_t kPingPongMaxSk = 2048, kPingPongPartMaxSk = 2560;
 constexpr double kRoundUs = 4.0, kTileUs = 1.78, kMergeUs = 8.0;
 constexpr double kKsRoundUs = 4.6, kKsTileUs = 2.1;
 static int fwd_kernel_choice(int64_t B, const FwdParams& p) {
@@ -663,7 +667,8 @@ static int fwd_kernel_choice(int64_t B, const FwdParams& p) {
   if (p.split_items > 0)
     other += rounds_us((int64_t)p.split_items * p.nsplit, (tiles + p.nsplit - 1) / p.nsplit) + kMergeUs;
   if (ks < other && (!p.seqused || ks_rounds == 1)) return 2;
-  return p.Sk <= kPingPongMaxSk ? 0 : 1;
+  const bool part = p.total_blocks % ncu != 0 && 4 * (int64_t)p.total_blocks < 7 * ncu;
+  return p.Sk <= (part ? kPingPongPartMaxSk : kPingPongMaxSk) ? 0 : 1;
 }
 
 // Which form of the one-wave kernel runs: the first-tile max (true) saves

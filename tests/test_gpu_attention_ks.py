@@ -162,3 +162,28 @@ def test_key_split_infinite_value(pkg, monkeypatch, Sk, key):
     assert torch.isposinf(out[..., 5]).all()
     out[..., 5] = want[..., 5]
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize(
+    "B,Sk,kernel",
+    [
+        (27, 2304, "pp"),  # 432 work items of 256 queries: 1.69 rounds of 256
+        (28, 2304, "1w"),  # 1.75
+        (16, 2304, "1w"),  # one whole round
+        (16, 2048, "pp"),
+        (32, 2049, "1w"),  # two
+    ],
+)
+def test_kernel_by_rounds(pkg, monkeypatch, B, Sk, kernel):
+    """Beyond 2048 keys the two-group kernel takes only calls that fill their last round in
+    part: the bits of the named kernel, not of the other."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("rounds are counted for 256 CUs")
+    g = torch.Generator(device="cuda").manual_seed(B)
+    q, k, v = (torch.randn(B, s, 16, 128, generator=g, device="cuda").to(BF) for s in (256, Sk, Sk))
+    out = pkg.attention(q, k, v)
+    forced = {}
+    for name in ("pp", "1w"):
+        monkeypatch.setenv("AA_FWD_KERNEL", name)
+        forced[name] = torch.equal(pkg.attention(q, k, v), out)
+    assert forced == {name: name == kernel for name in forced}
