@@ -637,14 +637,23 @@ static int dkdv_kernel_choice() {
 // split kernel of attn_bwd_dq_ks.hip, 64 queries per workgroup, instead of
 // dq_kernel: none, the last ones that dq_kernel would run as a partial round,
 // or all (a call of less than one round). Estimated time in us of a round of
-// each is a constant plus its 64-key tiles; the constants are fits to
-// graph-timed calls on MI355X (16 heads). The whole backward, dq_kernel ->
-// key split: B=1 256 tokens 27.3 -> 20.5, 512 45.5 -> 34.0, 1024 70.9 ->
-// 54.6, 2048 128.5 -> 122, 512 x 4096 keys 147 -> 87; where the rule turns it
-// down: 2304 tokens 190 against 202, B=2 1024 x 512 keys 61.8 against 63.2.
+// each is a constant plus its 64-key tiles. Where the key-split kernel runs one
+// round, the estimated difference was within 4 us of the measured one for calls
+// up to 1024 tokens (graph-timed, MI355X); its second round is over-estimated
+// (an empty CU share and a faster clock), by 7 us at 1280 tokens and 14 at 1545.
+// The whole backward, dq_kernel -> key split: B=1 x 16 heads 256 tokens 27.0 ->
+// 20.3, 512 45.9 -> 34.1, 1024 71.3 -> 53.3, 2048 129.1 -> 114.8, 512 x 4096
+// keys 150 -> 77.6; where the rule turns it down: 2304 tokens 165.4 against
+// 170.4, B=2 1024 x 512 keys 61.1 against 61.3, but 1545 tokens 92.4 against
+// 82.3. With no more than one key tile, which leaves two of its four waves
+// without keys, it takes calls of more than 128 queries (36 x 36 14.2 against
+// 15.4 us, 87 x 58 15.9 against 16.5, but 164 x 63 at B=2 19.3 against 18.2 and
+// 284 x 58 at 4 heads 23.1 against 20.1) and no tails, which cost a launch more
+// (B=4 2199 x 53 68.6 against 71.7; two tiles and 64 tail items tie).
 // AA_DQ_KERNEL=2g|ks forces none or all; -1 for another value.
 constexpr double kDqRoundUs = 7.5, kDqTileUs = 1.9, kDqKsRoundUs = 4.3, kDqKsTileUs = 3.6;
-static int64_t dq_ks_items(int64_t items, int64_t Sk) {
+constexpr int64_t kDqKsTileMinSq = 129;
+static int64_t dq_ks_items(int64_t items, int64_t Sq, int64_t Sk) {
   const char* e = std::getenv("AA_DQ_KERNEL");
   if (e && *e) {
     const std::string v = e;
@@ -653,6 +662,7 @@ static int64_t dq_ks_items(int64_t items, int64_t Sk) {
     return -1;
   }
   const int64_t ncu = std::max(device_cu_count(), 1), rem = items % ncu, tiles = (Sk + kT - 1) / kT;
+  if (tiles <= 1 && (Sq < kDqKsTileMinSq || items > ncu)) return 0;
   const double whole = kDqRoundUs + kDqTileUs * (double)tiles;
   const double split = (double)((4 * rem + ncu - 1) / ncu) *
                        (kDqKsRoundUs + kDqKsTileUs * (double)((tiles + 3) / 4));
@@ -701,7 +711,7 @@ extern "C" int aa_attn_bwd(const aa_attn_bwd_args* a, void* workspace, size_t wo
   if (dkdv_which < 0) return fail(AA_EINVAL, "AA_DKDV_KERNEL must be 1w or 2role");
   const int64_t nqitem = (a->Sq + bwd::kQueriesPerWg - 1) / bwd::kQueriesPerWg;
   const int64_t dq_items = a->B * a->H * nqitem;
-  const int64_t dq_ks = bwd::dq_ks_items(dq_items, a->Sk);
+  const int64_t dq_ks = bwd::dq_ks_items(dq_items, a->Sq, a->Sk);
   if (dq_ks < 0) return fail(AA_EINVAL, "AA_DQ_KERNEL must be 2g or ks");
   const bwd::WsLayout wl = bwd::ws_layout(a->B, a->Sq, a->Sk, a->H);
   const size_t need = aa_attn_bwd_workspace(a->B, a->Sq, a->Sk, a->H, a->hd);

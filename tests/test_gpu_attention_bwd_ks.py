@@ -81,3 +81,25 @@ def test_dq_kernel_env_rejects_unknown_value(pkg, monkeypatch):
     monkeypatch.setenv("AA_DQ_KERNEL", "zz")
     with pytest.raises(ValueError, match="AA_DQ_KERNEL"):
         torch.ops.anima_flat.fa_bwd(dout, q, k, v, out, lse)
+
+
+@pytest.mark.parametrize(
+    "Sq,Sk,H,kernel",
+    [
+        (128, 64, 16, "2g"),
+        (129, 64, 16, "ks"),
+        (128, 65, 16, "ks"),
+        (20, 60, 16, "2g"),
+        (200, 64, 260, "2g"),  # a tail of 4 items behind a whole round
+    ],
+)
+def test_dq_kernel_by_size(pkg, monkeypatch, Sq, Sk, H, kernel):
+    """Short calls and tails of one key tile keep the two-group kernel: dQ has its bits, not the other's
+    (with up to 32 keys the two sum the same products in the same order: no such case here)."""
+    q, k, v, dout = _inputs(1, Sq, Sk, H, 70)
+    dq = _gpu_backward(q, k, v, dout)[0]
+    forced = {}
+    for name in ("2g", "ks"):
+        monkeypatch.setenv("AA_DQ_KERNEL", name)
+        forced[name] = torch.equal(_gpu_backward(q, k, v, dout)[0], dq)
+    assert forced == {name: name == kernel for name in forced}
