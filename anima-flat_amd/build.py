@@ -4,7 +4,8 @@ extension _anima_torch.so (csrc/torch_ops.cpp, host code only) with g++.
 Objects go to `_build/` next to this file and the libraries to this directory,
 where `_lib.py` and `_native.py` load them from. Every source compiles in
 parallel; nothing is cached between calls (the caller asks for a build, so it
-gets one).
+gets one). The library needs hipcc only; without torch, its headers or g++ the
+extension is left out, with a warning.
 
 Run as a script to build: ``python anima-flat_amd/build.py``.
 """
@@ -16,6 +17,7 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import warnings
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -147,9 +149,12 @@ def _torch_commands() -> tuple[list[str], list[str]]:
     return compile_cmd, link_cmd
 
 
-def build(verbose: bool = False) -> Path:
+def build(verbose: bool = False, require_torch_ext: bool = False) -> Path:
     """Compile every source, link libanima_attn.so, the calibration library
-    libanima_calib.so and the torch extension; returns the attention library's path."""
+    libanima_calib.so and the torch extension; returns the attention library's path.
+
+    An extension that cannot be built raises with `require_torch_ext`. Otherwise it is
+    reported and left out, an earlier one with it: that was linked for another library."""
     cc = hipcc()
     SGPR_SPILL_WARNINGS.clear()
     BUILD.mkdir(exist_ok=True)
@@ -161,10 +166,20 @@ def build(verbose: bool = False) -> Path:
             objs.append(str(obj))
         cmds.append([cc, *DEVICE_FLAGS, *SOURCE_FLAGS.get(src, []), RESOURCE_REMARK, "-c",
                      str(CSRC / src), "-o", str(obj)])
-    torch_compile, torch_link = _torch_commands()
-    cmds.append(torch_compile)
-    workers = max(1, min(len(cmds), os.cpu_count() or 1, 8))
+    torch_link: list[str] = []
+    torch_error: Exception | None = None
+
+    def compile_torch() -> None:
+        nonlocal torch_link, torch_error
+        try:
+            torch_compile, torch_link = _torch_commands()
+            _run(torch_compile)
+        except (ImportError, OSError, RuntimeError) as e:
+            torch_error = e
+
+    workers = max(1, min(len(cmds) + 1, os.cpu_count() or 1, 8))
     with ThreadPoolExecutor(workers) as pool:
+        pool.submit(compile_torch)
         for cmd, _ in zip(cmds, pool.map(_run, cmds)):
             if verbose:
                 print(" ".join(cmd), flush=True)
@@ -178,8 +193,18 @@ def build(verbose: bool = False) -> Path:
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(ctmp),
           str(BUILD / (Path(CALIB_SOURCE).stem + ".o"))])
     os.replace(ctmp, CALIB_LIB_PATH)
-    _run(torch_link)
-    os.replace(str(TORCH_LIB_PATH) + ".tmp", TORCH_LIB_PATH)
+    if torch_error is None:
+        try:
+            _run(torch_link)
+            os.replace(str(TORCH_LIB_PATH) + ".tmp", TORCH_LIB_PATH)
+        except (OSError, RuntimeError) as e:
+            torch_error = e
+    if torch_error is not None:
+        TORCH_LIB_PATH.unlink(missing_ok=True)
+        if require_torch_ext:
+            raise torch_error
+        warnings.warn(f"{TORCH_LIB_PATH.name} is left out (the torch ops go through Python): {torch_error}",
+                      RuntimeWarning, stacklevel=2)
     return LIB_PATH
 
 
