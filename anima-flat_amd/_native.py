@@ -33,6 +33,15 @@ _ext = None
 _missing = False
 
 
+def _version_error(module) -> str | None:
+    """Why the extension must not be used: the argument structs it was compiled with, the
+    library it is linked to and this package have to agree on the ABI version."""
+    versions = module.abi_version(), module.library_abi_version(), _lib.ABI_VERSION
+    if len(set(versions)) == 1:
+        return None
+    return "was compiled for ABI version {}, runs on a library of {} and is called by a package of {}".format(*versions)
+
+
 def _load():
     """The extension module, or None (reported once) when it is not built."""
     global _ext, _missing
@@ -47,9 +56,9 @@ def _load():
         spec = importlib.util.spec_from_file_location("_anima_torch", EXT_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
-        if module.abi_version() != _lib.ABI_VERSION:
-            raise RuntimeError(
-                f"{EXT_PATH.name} is linked to ABI version {module.abi_version()}, expected {_lib.ABI_VERSION}")
+        error = _version_error(module)
+        if error is not None:
+            raise RuntimeError(f"{EXT_PATH.name} {error}")
         _ext = module
     return _ext
 

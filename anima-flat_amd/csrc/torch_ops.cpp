@@ -614,5 +614,7 @@ void attach(const std::string& qualname, pybind11::function impl) {
 
 PYBIND11_MODULE(_anima_torch, m) {
   m.def("attach", &attach, "Native dispatcher kernels for one op of the package");
-  m.def("abi_version", &aa_abi_version, "Of the libanima_attn.so it is linked to");
+  // What this file's argument structs are laid out for; the library may be newer.
+  m.def("abi_version", [] { return AA_ABI_VERSION; }, "Of the header it was compiled with");
+  m.def("library_abi_version", &aa_abi_version, "Of the libanima_attn.so it is linked to");
 }

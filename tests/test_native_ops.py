@@ -4,10 +4,13 @@ results, autograd behaviour and errors, whichever of the two a call reaches."""
 from __future__ import annotations
 
 import importlib
+import re
+import types
 
 import pytest
 import torch
 
+import __graft_entry__
 from oracle import attn_oracle as ref
 
 BF = torch.bfloat16
@@ -114,3 +117,31 @@ def test_weights_in_another_dtype(pkg):
     want = pkg.qkv_norm_rope(qkv, qw, kw, cos, sin, 2, 1e-6)
     got = pkg.qkv_norm_rope(qkv, *(t.to(BF) for t in (qw, kw, cos, sin)), 2, 1e-6)
     assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
+# ------------------------------------------------- loading the extension --
+
+
+@pytest.fixture
+def native(pkg, monkeypatch):
+    """anima_flat_amd._native as at its import, to be loaded again."""
+    module = importlib.import_module("anima_flat_amd._native")
+    if not (module.EXT_PATH.exists() and pkg._lib.LIB_PATH.exists()):
+        pytest.skip("not built (run __graft_entry__.build())")
+    monkeypatch.setattr(module, "_ext", None)
+    monkeypatch.setattr(module, "_missing", False)
+    return module
+
+
+def test_extension_version_is_the_headers(native):
+    text = (__graft_entry__.ROOT / "include" / "anima_attn.h").read_text()
+    ext = native._load()
+    assert ext.abi_version() == int(re.search(r"#define AA_ABI_VERSION (\d+)", text)[1])
+    assert ext.abi_version() == ext.library_abi_version()
+
+
+@pytest.mark.parametrize("compiled,library", [(2, 3), (3, 4), (4, 4)])
+def test_another_versions_extension_is_refused(native, compiled, library):
+    """Structs of another layout than the library's, also where library and package agree."""
+    module = types.SimpleNamespace(abi_version=lambda: compiled, library_abi_version=lambda: library)
+    assert f"compiled for ABI version {compiled}" in native._version_error(module)
