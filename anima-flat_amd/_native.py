@@ -5,7 +5,7 @@ that call libanima_attn.so straight from C++; `impl`, the op's Python function,
 stays the kernel of every other dispatch key and takes the calls the native
 kernels hand back (copies, other dtypes, errors). The extension is built with
 the library (build.py); without it the ops run the same HIP kernels through
-Python, which is reported once.
+Python, which is reported once; so they do if it does not load.
 """
 
 from __future__ import annotations
@@ -33,6 +33,14 @@ _ext = None
 _missing = False
 
 
+def _unusable(why: str) -> None:
+    """Say once that this process calls every op through Python, and why."""
+    global _missing
+    _missing = True
+    warnings.warn(f"{EXT_PATH.name} {why}: every op call of this process goes through Python "
+                  "(`python anima-flat_amd/build.py` builds it)", RuntimeWarning, stacklevel=5)
+
+
 def _version_error(module) -> str | None:
     """Why the extension must not be used: the argument structs it was compiled with, the
     library it is linked to and this package have to agree on the ABI version."""
@@ -43,22 +51,26 @@ def _version_error(module) -> str | None:
 
 
 def _load():
-    """The extension module, or None (reported once) when it is not built."""
+    """The extension module, or None (reported once) when it is not built or does not load
+    (another torch's, a library it cannot find)."""
     global _ext, _missing
     if _ext is None and not _missing:
-        if not (EXT_PATH.exists() and _lib.LIB_PATH.exists()):
+        if not _lib.LIB_PATH.exists():
             _missing = True
-            if _lib.LIB_PATH.exists():
-                warnings.warn(
-                    f"{EXT_PATH.name} is not built (run `python anima-flat_amd/build.py`): "
-                    "every op call goes through Python", RuntimeWarning, stacklevel=3)
             return None
-        spec = importlib.util.spec_from_file_location("_anima_torch", EXT_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        error = _version_error(module)
+        if not EXT_PATH.exists():
+            _unusable("is not built")
+            return None
+        try:
+            spec = importlib.util.spec_from_file_location("_anima_torch", EXT_PATH)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            error = _version_error(module)
+        except (ImportError, OSError, AttributeError) as e:
+            error = f"does not load ({e})"
         if error is not None:
-            raise RuntimeError(f"{EXT_PATH.name} {error}")
+            _unusable(error)
+            return None
         _ext = module
     return _ext
 

@@ -5,7 +5,11 @@ from __future__ import annotations
 
 import importlib
 import re
+import shutil
+import subprocess
+import sys
 import types
+import warnings
 
 import pytest
 import torch
@@ -145,3 +149,34 @@ def test_another_versions_extension_is_refused(native, compiled, library):
     """Structs of another layout than the library's, also where library and package agree."""
     module = types.SimpleNamespace(abi_version=lambda: compiled, library_abi_version=lambda: library)
     assert f"compiled for ABI version {compiled}" in native._version_error(module)
+
+
+def test_missing_extension_is_reported_once(native, monkeypatch, tmp_path):
+    monkeypatch.setattr(native, "EXT_PATH", tmp_path / "_anima_torch.so")
+    with pytest.warns(RuntimeWarning, match="is not built"):
+        assert native._load() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert native._load() is None
+
+
+def test_import_with_an_extension_that_does_not_load(native, tmp_path):
+    """The package imports, says so and keeps its Python ops (an extension of another torch)."""
+    copy = tmp_path / "anima-flat_amd"
+    shutil.copytree(__graft_entry__.PKG_DIR, copy, ignore=shutil.ignore_patterns("_build", "csrc", "__pycache__"))
+    (copy / "_anima_torch.so").write_bytes(b"no shared object")
+    code = f"""
+import pathlib, sys, warnings
+sys.path.insert(0, {str(__graft_entry__.ROOT)!r})
+import torch, __graft_entry__ as g
+g.PKG_DIR = pathlib.Path({str(copy)!r})
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    pkg = g.load_package()
+assert pkg.__file__.startswith({str(copy)!r})
+assert [w for w in seen if "does not load" in str(w.message)] and len(seen) == 1, [str(w.message) for w in seen]
+assert pkg._lib.available() and not pkg.use_fa4(torch.empty(1, dtype=torch.bfloat16))
+assert torch.ops.anima_flat.fa_fwd(*[torch.empty(1, 2, 1, 128, dtype=torch.bfloat16, device="meta")] * 3)[0].is_meta
+"""
+    proc = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert proc.returncode == 0, proc.stderr
