@@ -139,6 +139,7 @@ class AttnBwdArgs(Structure):
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+on_load: list = []  # called, in order, once the library is loaded
 
 
 def lib() -> ctypes.CDLL:
@@ -164,6 +165,8 @@ def lib() -> ctypes.CDLL:
                     f"{LIB_PATH.name} has ABI version {version}, expected {ABI_VERSION}"
                 )
             _lib = handle
+            while on_load:
+                on_load.pop(0)()
     return _lib
 
 

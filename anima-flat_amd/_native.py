@@ -56,7 +56,9 @@ def _load():
     global _ext, _missing
     if _ext is None and not _missing:
         if not _lib.LIB_PATH.exists():
+            # Nothing to call either: said when the library is there in the end.
             _missing = True
+            _lib.on_load.append(lambda: _unusable("was not built when the package was imported"))
             return None
         if not EXT_PATH.exists():
             _unusable("is not built")

@@ -134,6 +134,7 @@ def native(pkg, monkeypatch):
         pytest.skip("not built (run __graft_entry__.build())")
     monkeypatch.setattr(module, "_ext", None)
     monkeypatch.setattr(module, "_missing", False)
+    monkeypatch.setattr(pkg._lib, "on_load", [])
     return module
 
 
@@ -158,6 +159,19 @@ def test_missing_extension_is_reported_once(native, monkeypatch, tmp_path):
     with warnings.catch_warnings():
         warnings.simplefilter("error")
         assert native._load() is None
+
+
+def test_library_built_after_the_import(pkg, native, monkeypatch, tmp_path):
+    """With nothing built there is nothing to report, until the library is there."""
+    built = pkg._lib.LIB_PATH
+    monkeypatch.setattr(pkg._lib, "LIB_PATH", tmp_path / "libanima_attn.so")
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert native._load() is None
+    monkeypatch.setattr(pkg._lib, "LIB_PATH", built)
+    monkeypatch.setattr(pkg._lib, "_lib", None)
+    with pytest.warns(RuntimeWarning, match="was not built when the package was imported"):
+        pkg._lib.lib()
 
 
 def test_import_with_an_extension_that_does_not_load(native, tmp_path):
