@@ -110,10 +110,129 @@ def test_errors_are_the_python_functions(pkg):
         pkg.attention(q.cpu(), k.cpu(), v.cpu())
 
 
+def _op_cases():
+    """Arguments of every op with native kernels, by qualified name: fp32 norm weights and
+    tables whose values bf16 holds exactly."""
+    q, k, v = _qkv()
+    g = torch.Generator().manual_seed(5)
+
+    def n(*shape):
+        return ref.bf16_normal(shape, g).cuda()
+
+    dout, x, dy = n(1, 70, 2, 128).to(BF), n(1, 40, 256).to(BF), n(1, 40, 2, 128).to(BF)
+    qkv, grads = n(1, 40, 768).to(BF), [n(1, 40, 2, 128).to(BF) for _ in range(3)]
+    qw, kw, cos, sin = n(128), n(128), n(40, 64), n(40, 64)
+    q384, k384, v384 = (n(1, 50, 2, 384).to(BF) for _ in range(3))
+    lens = torch.tensor([33], dtype=torch.int32, device="cuda")
+    out, lse = torch.ops.anima_flat.fa_fwd(q, k, v)
+    eps = 1e-6
+    return {
+        "anima_flat::fa_fwd": (q, k, v),
+        "anima_flat::fa_fwd_nolse": (q, k, v),
+        "anima_flat::fa_fwd_k": (q, k, v, lens),
+        "anima_flat::fa_bwd": (dout, q, k, v, out, lse),
+        "anima_flat_amd::fa_fwd_k_ctx": (q, k, v, lens, torch.log(90.0 - lens)),
+        "anima_flat_amd::attend_d384": (q384, k384, v384),
+        "anima_flat::qkv_norm_rope": (qkv, qw, kw, cos, sin, 2, eps),
+        "anima_flat::qkv_norm_rope_v": (qkv, qw, kw, cos, sin, 2, eps),
+        "anima_flat::qkv_norm_rope_bwd": (qkv, *grads, qw, kw, cos, sin, 2, eps),
+        "anima_flat::head_norm": (x, qw, 2, eps),
+        "anima_flat::head_norm_bwd": (x, dy, qw, 2, eps),
+        "anima_flat_amd::qkv_proj_norm_rope": (x, n(768, 256).to(BF), qw, kw, cos, sin, 2, eps),
+        "anima_flat_amd::proj_head_norm": (x, n(256, 256).to(BF), qw, 2, eps),
+        "anima_flat_amd::kv_proj_norm": (x, n(512, 256).to(BF), kw, 2, eps),
+    }
+
+
+def _python_function(qualname):
+    """The function that op `qualname` was registered with."""
+    for name in ("attention", "vae", "kernels.rope", "kernels.proj"):
+        for op in vars(importlib.import_module(f"anima_flat_amd.{name}")).values():
+            if isinstance(op, torch.library.CustomOpDef) and op._qualname == qualname:
+                return op._init_fn
+    raise AssertionError(qualname)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("weights", [torch.float32, BF])
+def test_python_functions_give_the_same_bits(pkg, proj, weights):
+    """What a call gets without the extension, for every op it serves, also where the Python
+    function converts norm weights and tables (each to a tensor that lives until the launch:
+    their values are the same, so are all bits but those of the weights' own gradients)."""
+    cases = _op_cases()
+    assert set(cases) == importlib.import_module("anima_flat_amd._native").NATIVE_OPS
+    for name, args in cases.items():
+        ns, op = name.split("::")
+        want = getattr(getattr(torch.ops, ns), op)(*args)
+        cast = args if name.split("::")[1].startswith("fa_") else [
+            a.to(weights) if isinstance(a, torch.Tensor) and a.dtype == torch.float32 else a for a in args]
+        got = _python_function(name)(*cast)
+        want, got = ([t] if isinstance(t, torch.Tensor) else list(t) for t in (want, got))
+        assert len(want) == len(got)
+        assert all(torch.equal(a.to(b.dtype), b) for a, b in zip(want, got)), name
+
+
+@pytest.mark.gpu
+def test_functional_transforms(pkg):
+    """vmap batches a call without gradients; functorch's derivatives and forward mode, which
+    no op here has, are refused and give no wrong result."""
+    import torch.autograd.forward_ad as fwad
+
+    q, k, v = _qkv()
+    want = pkg.attention(q, k, v)
+    assert torch.equal(torch.func.vmap(pkg.attention)(q[None], k[None], v[None])[0], want)
+    leaf = q.clone().requires_grad_()
+    scale = torch.arange(1.0, 3.0, device="cuda").to(BF)
+    batched = torch.func.vmap(lambda x: pkg.attention(leaf, k, v) * x)(scale)  # of a constant
+    assert batched.requires_grad and torch.equal(batched[1], 2 * want)
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        torch.func.grad(lambda a: pkg.attention(a, k, v).float().sum())(q)
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        torch.func.vjp(lambda a: pkg.head_norm(a, torch.ones(128, device="cuda"), 2), q.flatten(2))
+    with fwad.dual_level(), pytest.raises(NotImplementedError, match="forward mode AD"):
+        pkg.attention(fwad.make_dual(leaf, torch.ones_like(q)), k, v)
+
+
+@pytest.mark.gpu
+def test_streams_and_threads(pkg):
+    """Calls from several threads, each on its own stream, forward and backward, with their
+    temporaries (converted weights, workspaces) in use at once: the bits of a call alone."""
+    import threading
+
+    g = torch.Generator().manual_seed(6)
+    qw, cos, sin = (ref.bf16_normal(s, g).to("cuda", BF) for s in ((128,), (300, 64), (300, 64)))
+    inputs = [ref.bf16_normal((1, 300, 3 * 512), g).to("cuda", BF) for _ in range(4)]
+
+    def step(x):
+        x = x.detach().requires_grad_()
+        q, k, v = pkg.qkv_norm_rope(x, qw, qw, cos, sin, 4, 1e-6)
+        out = pkg.attention(q, k, v)
+        return out, torch.autograd.grad(out.float().pow(2).sum(), x)[0]
+
+    want = [step(x) for x in inputs]
+    torch.cuda.synchronize()
+    got = [None] * len(inputs)
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(10):
+                got[i] = step(inputs[i])
+        stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(inputs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(want, got):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
 @pytest.mark.gpu
 def test_weights_in_another_dtype(pkg):
     """bf16 norm weights and tables are converted, each to a tensor of its own that lives
-    until the launch."""
+    until the launch (test_python_functions_give_the_same_bits: on the Python path)."""
     g = torch.Generator().manual_seed(4)
     qkv = ref.bf16_normal((1, 40, 3 * 256), g).to("cuda", BF)
     qw, kw = (ref.bf16_normal((128,), g).cuda() for _ in range(2))
