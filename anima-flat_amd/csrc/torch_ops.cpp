@@ -487,28 +487,31 @@ struct Plain {
   }
 };
 
+// One output: the LSE, which has no derivative, is handed past the node (a node
+// with an output marked as such cannot be traced by compiled autograd).
 struct FaFwd : torch::autograd::Function<FaFwd> {
   static constexpr bool is_traceable = true;
-  static variable_list forward(AutogradContext* ctx, CT q, CT k, CT v) {
-    auto [out, lse] = op_fa_fwd().below(q, k, v);
-    ctx->mark_non_differentiable({lse});
-    // The backward never reads the LSE's gradient: no zeros are made for it.
+  static Tensor forward(AutogradContext* ctx, CT q, CT k, CT v, Tensor* lse) {
+    Tensor out;
+    std::tie(out, *lse) = op_fa_fwd().below(q, k, v);
     ctx->set_materialize_grads(false);
-    ctx->save_for_backward({q, k, v, out, lse});
-    return {out, lse};
+    ctx->save_for_backward({q, k, v, out, *lse});
+    return out;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
-    if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
-    return as_list(op_fa_bwd()(grads[0], s[0], s[1], s[2], s[3], s[4]));
+    if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
+    variable_list g = as_list(op_fa_bwd()(grads[0], s[0], s[1], s[2], s[3], s[4]));
+    g.emplace_back();
+    return g;
   }
 };
 
 T2 fa_fwd_autograd(CT q, CT k, CT v) {
   if (!needs_grad(q, k, v)) return op_fa_fwd().below(q, k, v);
-  T2 r;
-  from_list(FaFwd::apply(q, k, v), r);
-  return r;
+  Tensor lse;
+  Tensor out = FaFwd::apply(q, k, v, &lse);
+  return {out, lse};
 }
 
 struct QkvNormRopeV : torch::autograd::Function<QkvNormRopeV> {

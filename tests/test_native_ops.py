@@ -13,6 +13,7 @@ import warnings
 
 import pytest
 import torch
+import torch._dynamo.compiled_autograd
 
 import __graft_entry__
 from oracle import attn_oracle as ref
@@ -191,6 +192,29 @@ def test_functional_transforms(pkg):
         torch.func.vjp(lambda a: pkg.head_norm(a, torch.ones(128, device="cuda"), 2), q.flatten(2))
     with fwad.dual_level(), pytest.raises(NotImplementedError, match="forward mode AD"):
         pkg.attention(fwad.make_dual(leaf, torch.ones_like(q)), k, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["attention", "head_norm", "prologue"])
+def test_compiled_autograd(pkg, path):
+    """torch.compile's tracing of the backward goes through the ops' autograd nodes."""
+    q, k, v = _qkv()
+    w, cos, sin = torch.ones(128, device="cuda"), *torch.randn(2, 70, 64, device="cuda")
+
+    def run(a):
+        if path == "attention":
+            return pkg.attention(a, k, v)
+        if path == "head_norm":
+            return pkg.head_norm(a.flatten(2), w, 2)
+        qkv = torch.cat([t.flatten(2) for t in (a, k[:, :70], v[:, :70])], -1)
+        return pkg.qkv_norm_rope(qkv, w, w, cos, sin, 2)[0]  # two outputs without a gradient
+
+    leaf = q.clone().requires_grad_()
+    run(leaf).float().pow(2).sum().backward()
+    want, leaf.grad = leaf.grad, None
+    with torch._dynamo.compiled_autograd._enable(torch.compile(backend="eager")):
+        run(leaf).float().pow(2).sum().backward()
+    assert torch.equal(leaf.grad, want)
 
 
 @pytest.mark.gpu
