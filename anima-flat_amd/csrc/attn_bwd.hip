@@ -268,7 +268,7 @@ void dkdv_kernel(Params p, int nkblk) {
   // its final M block; no DMA is in flight).
   if (rec >= 0) {
     // Partial accumulators, 16 coalesced 1 KB stores per wave: float4 j of
-    // lane l at ((logical * 8 + wave) * 16 + j) * 64 + l.
+    // lane l at ((rec * 8 + wave) * 16 + j) * 64 + l.
     f32x4* dst = reinterpret_cast<f32x4*>(p.part) + ((int64_t)rec * kDkWaves + wave) * 16 * 64 + lane;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -701,10 +701,8 @@ extern "C" int aa_attn_bwd(const aa_attn_bwd_args* a, void* workspace, size_t wo
                               a->out_stride,  a->dq_stride, a->dk_stride, a->dv_stride};
   for (const int64_t* s : strides)
     if (!bwd::stride_ok(s)) return fail(AA_EINVAL, "attn_bwd: strides must be multiples of 8");
-  // The tile DMA addresses rows by a 32-bit unsigned per-lane byte offset (up
-  // to 7 rows past a scalar row base).
   for (const int64_t* s : {a->q_stride, a->dout_stride, a->k_stride, a->v_stride})
-    if (s[1] < 0 || s[1] >= (1 << 24))
+    if (s[1] < 0 || s[1] >= kMaxRowStride)
       return fail(AA_EUNSUPPORTED, "attn_bwd: q / dout / k / v sequence strides must be in [0, 2^24) elements");
   if (!(a->softmax_scale > 0.f)) return fail(AA_EINVAL, "attn_bwd: softmax_scale must be > 0");
   const int dkdv_which = bwd::dkdv_kernel_choice();

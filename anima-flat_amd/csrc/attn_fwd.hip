@@ -534,12 +534,9 @@ static int prepare(const aa_attn_fwd_args* a, FwdParams& p) {
   if (a->ln_pad && !a->seqused_k) return fail(AA_EINVAL, "attn_fwd: ln_pad needs seqused_k");
   if (!(a->softmax_scale > 0.f) || !std::isfinite(a->softmax_scale))
     return fail(AA_EINVAL, "attn_fwd: softmax_scale must be positive and finite");
-  // The K/V tile DMA addresses rows by a 32-bit unsigned per-lane byte
-  // offset (up to 7 rows past a scalar row base): the stride must be
-  // non-negative and small enough.
-  if (a->k_stride[1] < 0 || a->v_stride[1] < 0 || a->k_stride[1] >= (1 << 24) ||
-      a->v_stride[1] >= (1 << 24))
-    return fail(AA_EUNSUPPORTED, "attn_fwd: key/value sequence stride must be in [0, 2^24) elements");
+  for (const int64_t rs : {a->k_stride[1], a->v_stride[1]})
+    if (rs < 0 || rs >= kMaxRowStride)
+      return fail(AA_EUNSUPPORTED, "attn_fwd: key/value sequence stride must be in [0, 2^24) elements");
 
   p.q = (const bf16*)a->q;
   p.k = (const bf16*)a->k;

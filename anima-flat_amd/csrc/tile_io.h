@@ -24,6 +24,12 @@ namespace aa {
 
 constexpr int kTileRows = 64;
 constexpr int kTileElems = kTileRows * 128;  // 16 KB of bf16
+// The tile DMA addresses a row by a 32-bit unsigned per-lane byte offset from a
+// scalar row base: up to 63 rows past it in the forward (31 in the key-split
+// dQ kernel, 7 in the other backward kernels), plus 128 columns. The entry
+// points refuse row strides (in elements) that are negative or not below this.
+constexpr int64_t kMaxRowStride = int64_t{1} << 24;
+static_assert(((kTileRows - 1) * kMaxRowStride + 128) * 2 <= int64_t{0xffffffff}, "32-bit row offsets");
 
 // Workgroup-wide DMA helpers ------------------------------------------------
 
@@ -138,10 +144,6 @@ __device__ __forceinline__ void dma16_sva_off(const void* sbase, uint32_t voff, 
   asm volatile("s_add_i32 m0, %2, %4\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(voff),
                "s"(sbu), "s"(base), "n"(kOff), "n"(kLds - kOff)
                : "memory", "m0", "scc");
-}
-// The same with the LDS destination as a pointer into __shared__ memory.
-__device__ __forceinline__ void dma16_sv(const void* sbase, uint32_t voff, const void* lds_dst) {
-  dma16_sva(sbase, voff, (uint32_t)(uintptr_t)(lds_void*)lds_dst);
 }
 
 // Chunk (0..7, within the block's 64 d) that DMA lane `lane` moves into its
