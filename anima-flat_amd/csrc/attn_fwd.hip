@@ -615,15 +615,21 @@ static int fwd_scratch(void** out) {
 //      of workgroups takes a constant plus its tiles per wave (the other
 //      kernels' tiles are up to 40% faster on a part-filled chip, whose clock
 //      is higher), and split items kMergeUs more for the partials' way through
-//      memory and the combine launch. The constants are fits to graph-timed
-//      calls on MI355X (16 heads, to within 10%). Measured against the other
-//      two: B=1 256 tokens 10.6 -> 8.8 us, 512 20.0 -> 10.5, 1024 22.0 ->
-//      14.3, B=2 1024 31.0 -> 27.3, 1024 x 512 keys 19.5 -> 11.0; where the
-//      rule turns it down: 1280 tokens 27.2 against 29.1, 1536 30.6 against
-//      31.9, B=2 700 22.8 against 23.4, 256 x 4096 keys 23.0 against 31.1,
-//      1024 x 64 keys 6.4 against 8.4. With key lengths, which only the device
-//      knows, one round at most (lengths 58 and 322 of 512, B=2: 300 queries
-//      16.3 -> 12.2, but 1000 21.4 -> 23.0).
+//      memory and the combine launch. The constants order the kernels; they are
+//      no fit of either (573 sizes, graph-timed on MI355X: the key-split
+//      estimate is 33% under to 31% over, the other 29% under to 39% over). Of
+//      822 calls the rule took the slower kernel for 5 (by 2.6-4.4%: 1035 x 481
+//      keys at 20 heads 21.3 against 20.4 us, B=2 530 x 95 15.7 against 15.3),
+//      and turned the key-split kernel down in 62 that it would have sped up
+//      (by up to 20%); estimates nearer to the times moved losses of 8-30% to
+//      other sizes. 16 heads, the others -> key split: 256 tokens 10.7 -> 8.4
+//      us, 512 19.9 -> 10.3, 1024 23.0 -> 15.1, B=2 1024 32.2 -> 28.5, 1024 x
+//      512 keys 20.1 -> 11.1; turned down: 1280 tokens 27.7 against 29.2, 1536
+//      32.2 against 32.9, 256 x 4096 keys 24.5 against 29.2, 1024 x 64 keys 6.6
+//      against 8.4, but B=2 700 23.4 against 22.6. With key lengths, which only
+//      the device knows, one round at most (lengths 58 and 322 of 512, B=2: 300
+//      queries 16.1 -> 10.5 us; two rounds of 1000 queries would now gain, too,
+//      21.2 against 19.4).
 //   else 0, the two-group kernel of attn_fwd_pp.hip, which hides more of a work
 //      item's fixed costs, up to kPingPongMaxSk keys, and beyond them 1, this
 //      file's one-wave-per-SIMD kernel. At 4096 queries, B = 1-2, the
